@@ -66,7 +66,7 @@ __host__ inline unsigned batch_grid(unsigned grid, uint32_t n)
 // the ensemble's step 6.63 -> 6.22 ms), seven without a sub-grid model, where eight loads
 // fewer populations in flight and ran slower (5.30 -> 5.92 ms).
 template <int SGS, bool IBB, int PASS, typename Real>
-constexpr int kBatch19MinWaves = (IBB || PASS != 1 || sizeof(Real) == 8) ? 1 : (SGS == 0 ? 8 : 7);
+constexpr int kBatch19MinWaves = sizeof(Real) == 8 ? 1 : ((IBB || PASS != 1) ? 5 : (SGS == 0 ? 8 : 7));
 
 template <typename S, typename Real, int SGS, int Q, bool IBB, int PASS, int COLL = COLL_CUMULANT>
 __global__ void __launch_bounds__(kBatchBlock)

@@ -31,6 +31,10 @@ struct L19 {
     static constexpr int cy[19] = {0, 0, 0, 1, -1, 0, 0, 1, -1, -1, 1, 0, 0, 0, 0, 1, -1, 1, -1};
     static constexpr int cz[19] = {0, 0, 0, 0, 0, 1, -1, 0, 0, 0, 0, 1, -1, -1, 1, 1, -1, -1, 1};
     __host__ __device__ static constexpr int opp(int q) { return q == 0 ? 0 : ((q & 1) ? q + 1 : q - 1); }
+    // diagonals with the x, y or z component flipped; the other directions reversed
+    static constexpr int mirx[19] = {0, 2, 1, 4, 3, 6, 5, 10, 9, 8, 7, 14, 13, 12, 11, 16, 15, 18, 17};
+    static constexpr int miry[19] = {0, 2, 1, 4, 3, 6, 5, 9, 10, 7, 8, 12, 11, 14, 13, 18, 17, 16, 15};
+    static constexpr int mirz[19] = {0, 2, 1, 4, 3, 6, 5, 8, 7, 10, 9, 13, 14, 11, 12, 17, 18, 15, 16};
 };
 
 template <typename Real>
@@ -170,30 +174,18 @@ __device__ inline long face_upwind(int q, long ic, int i, int j, int k, int nx, 
     return (long)s;
 }
 
-// kernel.cl:105-326 reflectOrMirrorQ as a table lookup: bounce-back partner, with
-// Symmetry faces flipping only the normal component of diagonal directions.
+// kernel.cl:105-326 reflectOrMirrorQ as table lookups: the bounce-back partner, with
+// Symmetry faces flipping only the normal component of diagonal directions -- of the first
+// of its axes, in the order x, y, z, whose code is Symmetry.  (Selects between constants once
+// q is: a face cell's pull takes its reflected slot from here.)
 __device__ inline int mirror_q(int q, int b1, int b2, int b3)
 {
-    if (q <= 6) return L19::opp(q);
-    int cx = L19::cx[q], cy = L19::cy[q], cz = L19::cz[q];
-    // flip the component normal to the first Symmetry face the reference tests
-    if (q <= 10) {  // xy diagonals: test b1 then b2
-        if (b1 == BC_SYMMETRY) cx = -cx;
-        else if (b2 == BC_SYMMETRY) cy = -cy;
-        else { cx = -cx; cy = -cy; }
-    } else if (q <= 14) {  // xz diagonals: b1 then b3
-        if (b1 == BC_SYMMETRY) cx = -cx;
-        else if (b3 == BC_SYMMETRY) cz = -cz;
-        else { cx = -cx; cz = -cz; }
-    } else {  // yz diagonals: b2 then b3
-        if (b2 == BC_SYMMETRY) cy = -cy;
-        else if (b3 == BC_SYMMETRY) cz = -cz;
-        else { cy = -cy; cz = -cz; }
-    }
-#pragma unroll
-    for (int p = 7; p < 19; p++)
-        if (L19::cx[p] == cx && L19::cy[p] == cy && L19::cz[p] == cz) return p;
-    return L19::opp(q);
+    int r = L19::opp(q);
+    if (q <= 6) return r;
+    if (L19::cz[q] != 0) r = (b3 == BC_SYMMETRY) ? L19::mirz[q] : r;
+    if (L19::cy[q] != 0) r = (b2 == BC_SYMMETRY) ? L19::miry[q] : r;
+    if (L19::cx[q] != 0) r = (b1 == BC_SYMMETRY) ? L19::mirx[q] : r;
+    return r;
 }
 
 // kernel.cl:1346-1395 cornerFlag
@@ -246,6 +238,14 @@ __device__ inline Real zouhe_sum(const Real *ft, int dir, bool lo)
     return s + Real(2) * t;
 }
 
+// c ? a : b of two values (a conditional on ft[] elements themselves would name one of two
+// addresses, and put ft[] in memory)
+template <typename T>
+__device__ inline T pick(bool c, T a, T b)
+{
+    return c ? a : b;
+}
+
 // Ladd moving-wall correction of the five populations entering through a face with
 // wall velocity (un, ut1, ut2) = (normal, first tangential, second tangential),
 // kernel.cl:1397-1512.  Written with value selects (never "if (lo) ft[a] else ft[b]")
@@ -287,37 +287,20 @@ struct Cell {
     int i, j, k;
 };
 
-// macro value of a neighbour: previous step's buffer; the cell itself: its new value
-template <typename Real>
-__device__ inline Real mac_at(const Real *old, long idx, long ic, Real self)
+// derivative of one component along an axis as kernel.cl:2275-2304 forms it: central inside;
+// on a face one-sided, with the cell's own value the new one (the reference reads it back
+// from the array it has just written); 0 for the z gradient at k = 0 (K19:2283, a - a) and on
+// a 2-D lattice.  Both neighbours are loaded, the cell itself in place of one outside the
+// lattice, and the form is chosen by selects: a branch per face and component left the nine
+// derivatives of a face wave waiting for memory one after another.
+template <int DIR, typename Real>
+__device__ inline Real grad_comp(const Real *old, Real self, uint32_t ic, int pos, int n, uint32_t stride)
 {
-    return idx == ic ? self : old[idx];
-}
-
-// one component of grad(u) as kernel.cl:2275-2304 forms it
-template <typename Real>
-__device__ inline Real grad_comp(const Real *old, Real self, long ic, int i, int j, int k, int nx, int ny, int nz,
-                                 int dir)
-{
-    const long sx = 1, sy = nx, sz = (long)nx * ny;
-    const long base = ic - i * sx - j * sy - k * sz;
-#define AT(ii, jj, kk) mac_at<Real>(old, base + (ii) * sx + (jj) * sy + (long)(kk) * sz, ic, self)
-    if (dir == 0)
-        return (i > 0 && i < nx - 1) ? Real(0.5) * (AT(i + 1, j, k) - AT(i - 1, j, k))
-             : (i == 0) ? AT(1, j, k) - AT(0, j, k)
-                        : AT(nx - 1, j, k) - AT(nx - 2, j, k);
-    if (dir == 1)
-        return (j > 0 && j < ny - 1) ? Real(0.5) * (AT(i, j + 1, k) - AT(i, j - 1, k))
-             : (j == 0) ? AT(i, 1, k) - AT(i, 0, k)
-                        : AT(i, ny - 1, k) - AT(i, ny - 2, k);
-    if (k > 0 && k < nz - 1) return Real(0.5) * (AT(i, j, k + 1) - AT(i, j, k - 1));
-    if (nz - 1 == 0) return Real(0);
-    if (k == 0) {
-        Real a = AT(i, j, 1);
-        return a - a;
-    }
-    return AT(i, j, nz - 1) - AT(i, j, nz - 2);
-#undef AT
+    const bool lo = (pos == 0), hi = (pos == n - 1);
+    const Real p = old[hi ? ic : ic + stride], m = old[lo ? ic : ic - stride];
+    const Real inside = Real(0.5) * (p - m);
+    if (DIR == 2) return n == 1 ? Real(0) : (lo ? p - p : (hi ? self - m : inside));
+    return lo ? p - self : (hi ? self - m : inside);
 }
 
 // kernel.cl:2267-2365 waleTauSGS (Cw = 0.325) from the velocity gradient
@@ -365,7 +348,11 @@ template <bool Interior, typename Real, int Q>
 __device__ inline Real wale_tau(const StepArgs<Real, Q> &a, long ic, int i, int j, int k, Real u, Real v, Real w)
 {
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    if (Interior && Q == 27 && i > 0 && i < nx - 1 && j > 0 && j < ny - 1 && k > 0 && k < nz - 1) {
+    // the choice is uniform over the wave (every active lane must allow the shorter form), so
+    // that a wave with a face cell runs one form and waits once for its loads
+    const bool yz_in = j > 0 && j < ny - 1 && k > 0 && k < nz - 1;
+    const bool all_yz_in = Interior && nx >= 3 && __ballot(!yz_in) == 0;
+    if (Q == 27 && all_yz_in && __ballot(!(i > 0 && i < nx - 1)) == 0) {
         // all six neighbours exist: central differences only, as grad_comp takes them there
         const uint32_t o = (uint32_t)ic * (uint32_t)sizeof(Real);
         const uint32_t dx = (uint32_t)sizeof(Real), dy = (uint32_t)nx * dx, dz = (uint32_t)ny * dy;
@@ -373,8 +360,8 @@ __device__ inline Real wale_tau(const StepArgs<Real, Q> &a, long ic, int i, int 
         return wale_from_grad<Real>(cdiff(U, o, dx), cdiff(U, o, dy), cdiff(U, o, dz), cdiff(V, o, dx), cdiff(V, o, dy),
                                     cdiff(V, o, dz), cdiff(W, o, dx), cdiff(W, o, dy), cdiff(W, o, dz));
     }
-    if (Interior && Q == 19 && nx >= 3 && j > 0 && j < ny - 1 && k > 0 && k < nz - 1) {
-        // (D3Q19, whose waves of x-face and interior cells run together) the y and z
+    if (all_yz_in) {
+        // (waves with x-face cells, and on D3Q19 every wave inside in y and z) the y and z
         // neighbours exist: central differences there, as grad_comp takes them; along x
         // central differences inside and, on an x face, grad_comp's one-sided difference with
         // the cell's own new velocity -- as a per-lane choice, so that such a wave runs one
@@ -392,15 +379,16 @@ __device__ inline Real wale_tau(const StepArgs<Real, Q> &a, long ic, int i, int 
         return wale_from_grad<Real>(ddx(U, u), cdiff(U, o, dy), cdiff(U, o, dz), ddx(V, v), cdiff(V, o, dy),
                                     cdiff(V, o, dz), ddx(W, w), cdiff(W, o, dy), cdiff(W, o, dz));
     }
-    Real dudx = grad_comp<Real>(a.u_o, u, ic, i, j, k, nx, ny, nz, 0);
-    Real dudy = grad_comp<Real>(a.u_o, u, ic, i, j, k, nx, ny, nz, 1);
-    Real dudz = grad_comp<Real>(a.u_o, u, ic, i, j, k, nx, ny, nz, 2);
-    Real dvdx = grad_comp<Real>(a.v_o, v, ic, i, j, k, nx, ny, nz, 0);
-    Real dvdy = grad_comp<Real>(a.v_o, v, ic, i, j, k, nx, ny, nz, 1);
-    Real dvdz = grad_comp<Real>(a.v_o, v, ic, i, j, k, nx, ny, nz, 2);
-    Real dwdx = grad_comp<Real>(a.w_o, w, ic, i, j, k, nx, ny, nz, 0);
-    Real dwdy = grad_comp<Real>(a.w_o, w, ic, i, j, k, nx, ny, nz, 1);
-    Real dwdz = grad_comp<Real>(a.w_o, w, ic, i, j, k, nx, ny, nz, 2);
+    const uint32_t c = (uint32_t)ic, sy = (uint32_t)nx, sz = sy * (uint32_t)ny;
+    auto row = [&](const Real *P, Real self, Real &dx, Real &dy, Real &dz) {
+        dx = grad_comp<0>(P, self, c, i, nx, 1u);
+        dy = grad_comp<1>(P, self, c, j, ny, sy);
+        dz = grad_comp<2>(P, self, c, k, nz, sz);
+    };
+    Real dudx, dudy, dudz, dvdx, dvdy, dvdz, dwdx, dwdy, dwdz;
+    row(a.u_o, u, dudx, dudy, dudz);
+    row(a.v_o, v, dvdx, dvdy, dvdz);
+    row(a.w_o, w, dwdx, dwdy, dwdz);
     return wale_from_grad<Real>(dudx, dudy, dudz, dvdx, dvdy, dvdz, dwdx, dwdy, dwdz);
 }
 
@@ -646,6 +634,34 @@ __device__ inline void collide_rr(Real *out, const Mom19<Real> &m, Real inv_rho,
     out[18] = h * (-M011 - M012) + dyz;
 }
 
+// The populations that enter through an outlet face, from the cell's and the inner
+// neighbour's own (previous) values: direction q at the min face, its opposite at the max
+// face (the two ends of an axis differ: a z outlet on a 2-D lattice is refused).  One select
+// of the direction per pair, so that the ten loads go out together.
+template <int DIR, typename S, typename Real>
+__device__ __forceinline__ void outlet19(Real *ft, const S *fs, uint32_t fstride, long ic, bool lo, long st, Real s)
+{
+    const uint32_t inner = (uint32_t)(lo ? ic + st : ic - st);
+    S fi[19], fc[19];
+#pragma unroll
+    for (int q = 1; q < 19; q++) {
+        if ((DIR == 0 ? L19::cx[q] : (DIR == 1 ? L19::cy[q] : L19::cz[q])) != 1) continue;
+        const int qd = lo ? q : L19::opp(q);
+        fi[q] = fs[pop_at<19, S>(qd, inner, fstride)];
+        fc[q] = fs[pop_at<19, S>(qd, (uint32_t)ic, fstride)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int q = 1; q < 19; q++) {
+        if ((DIR == 0 ? L19::cx[q] : (DIR == 1 ? L19::cy[q] : L19::cz[q])) != 1) continue;
+        const int qo = L19::opp(q);
+        const Real v = s * Codec<S, Real, 19>::load(&fi[q], q, w19<Real>(q)) +
+                       (Real(1) - s) * Codec<S, Real, 19>::load(&fc[q], q, w19<Real>(q));
+        ft[q] = pick(lo, v, ft[q]);
+        ft[qo] = pick(lo, ft[qo], v);
+    }
+}
+
 // Boundary handling of a domain-face cell: streaming with walls, then the face
 // conditions in the reference's order (kernel.cl:3581-3592).
 // xonly = false: every direction is streamed here.  xonly = true: a cell on an x face (and
@@ -659,22 +675,49 @@ __device__ __forceinline__ void face_cell(const Step19Args<Real> &a, Real *ft, u
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const S *fs = (const S *)a.fsrc;
     const int b1 = flag_code(fl, F_B1_SHIFT), b2 = flag_code(fl, F_B2_SHIFT), b3 = flag_code(fl, F_B3_SHIFT);
-    const bool sym = (b1 == BC_SYMMETRY || b2 == BC_SYMMETRY || b3 == BC_SYMMETRY);
-    Real Fx = 0, Fy = 0, Fz = 0;  // wall momentum of this step's domain-face links
     const int xs = (i == 0) ? 1 : -1;
-    if (!xonly) ft[0] = Codec<S, Real, 19>::load(fs + pop_at<19, S>(0, (uint32_t)ic, a.fstride), 0, w19<Real>(0));
+    // Every direction has exactly one source -- the upwind cell, or across a wall the cell's own
+    // reflected slot -- so its address is selected and all loads go out together.  A branch
+    // per direction with a load in either arm made a face wave wait for memory 18 times in a
+    // row, which bounds small lattices: with the velocity gradient of wale_tau likewise, a
+    // 32^3 FP32 cavity went from 14.5 to 9.8 us per step, 64^3 FP64 from 27.5 to 20 us, 60
+    // FP16 lattices of edge 24-96 from 0.81 to 0.70 ms.
+    S raw[19];
+    if (!xonly) {
+        // (each address right before its load: computed ahead of the loads, 18 64-bit addresses
+        // would not fit the registers beside the populations)
+        raw[0] = fs[pop_at<19, S>(0, (uint32_t)ic, a.fstride)];
 #pragma unroll
-    for (int q = 1; q < 19; q++) {
-        if (xonly && L19::cx[q] != xs) continue;
-        long src = face_upwind(q, ic, i, j, k, nx, ny, nz, b1, b2, b3);
-        if (src >= 0) {
-            ft[q] = Codec<S, Real, 19>::load(fs + pop_at<19, S>(q, (uint32_t)src, a.fstride), q, w19<Real>(q));
-        } else {
-            int qb = sym ? mirror_q(q, b1, b2, b3) : L19::opp(q);
-            ft[q] = Codec<S, Real, 19>::load(fs + pop_at<19, S>(qb, (uint32_t)ic, a.fstride), qb, w19<Real>(qb));
-            Fx += Real(-2) * ft[q] * Real(L19::cx[q]);
-            Fy += Real(-2) * ft[q] * Real(L19::cy[q]);
-            Fz += Real(-2) * ft[q] * Real(L19::cz[q]);
+        for (int q = 1; q < 19; q++) {
+            const long src = face_upwind(q, ic, i, j, k, nx, ny, nz, b1, b2, b3);
+            const size_t own = pop_at<19, S>(mirror_q(q, b1, b2, b3), (uint32_t)ic, a.fstride);
+            const size_t up = pop_at<19, S>(q, (uint32_t)src, a.fstride);
+            raw[q] = fs[src < 0 ? own : up];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < 19; q++) ft[q] = Codec<S, Real, 19>::load(&raw[q], q, w19<Real>(q));
+    } else {
+        // the five directions that cross the cell's x face: q with c_x = +1 at i = 0, its
+        // opposite at i = nx - 1 (j and k are interior: no other face is crossed)
+        const bool lo = (xs == 1), wall = is_wall_code(b1);
+#pragma unroll
+        for (int q = 1; q < 19; q++) {
+            if (L19::cx[q] != 1) continue;
+            const int qo = L19::opp(q);
+            const uint32_t src = (uint32_t)(ic - (lo ? a.off[q] : a.off[qo]) + xs * nx);
+            const int qb = lo ? mirror_q(q, b1, b2, b3) : mirror_q(qo, b1, b2, b3);
+            const size_t own = pop_at<19, S>(qb, (uint32_t)ic, a.fstride);
+            const size_t up = pop_at<19, S>(lo ? q : qo, src, a.fstride);
+            raw[q] = fs[wall ? own : up];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 1; q < 19; q++) {
+            if (L19::cx[q] != 1) continue;
+            const Real v = Codec<S, Real, 19>::load(&raw[q], q, w19<Real>(q));
+            ft[q] = pick(lo, v, ft[q]);
+            ft[L19::opp(q)] = pick(lo, ft[L19::opp(q)], v);
         }
     }
     const int corner = corner_flag(b3, i, j, k, nx, ny, nz);
@@ -738,6 +781,16 @@ __device__ __forceinline__ void face_cell(const Step19Args<Real> &a, Real *ft, u
     // wallFunctionBC, kernel.cl:1654-1924 (stationary wall, tangential slip velocity)
     if (corner == 0 && (b1 == BC_WALLFUNCTION || b2 == BC_WALLFUNCTION || b3 == BC_WALLFUNCTION)) {
         const Real nu = (Real(1) / omega - Real(0.5)) / Real(3);
+        // wall momentum of this step's domain-face links (off the corners a cell lies on one
+        // wall face, so no condition above has changed these populations)
+        Real Fx = 0, Fy = 0, Fz = 0;
+#pragma unroll
+        for (int q = 1; q < 19; q++)
+            if (face_upwind(q, ic, i, j, k, nx, ny, nz, b1, b2, b3) < 0) {
+                Fx += Real(-2) * ft[q] * Real(L19::cx[q]);
+                Fy += Real(-2) * ft[q] * Real(L19::cy[q]);
+                Fz += Real(-2) * ft[q] * Real(L19::cz[q]);
+            }
 #pragma unroll
         for (int dir = 0; dir < 3; dir++) {
             const int code = dir == 0 ? b1 : (dir == 1 ? b2 : b3);
@@ -776,24 +829,9 @@ __device__ __forceinline__ void face_cell(const Step19Args<Real> &a, Real *ft, u
     // outflowBC, kernel.cl:2005-2097: convective outlet with the cell's last velocity
     if (b1 == BC_OUTLET || b2 == BC_OUTLET || b3 == BC_OUTLET) {
         const Real is3 = Real(0.57735026918962576);
-        const Real uo = a.u_o[ic], vo = a.v_o[ic], wo = a.w_o[ic];
-#pragma unroll
-        for (int q = 1; q < 19; q++) {
-            const int cx = L19::cx[q], cy = L19::cy[q], cz = L19::cz[q];
-#define OUTF(cond, inner, un)                                                                          \
-    if (cond) {                                                                                        \
-        const Real fi = Codec<S, Real, 19>::load(fs + pop_at<19, S>(q, (uint32_t)(inner), a.fstride), q, w19<Real>(q)); \
-        const Real fc = Codec<S, Real, 19>::load(fs + pop_at<19, S>(q, (uint32_t)ic, a.fstride), q, w19<Real>(q)); \
-        ft[q] = (is3 - (un)) * fi + (Real(1) - (is3 - (un))) * fc;                                      \
-    }
-            OUTF(i == 0 && b1 == BC_OUTLET && cx == 1, ic + 1, uo)
-            OUTF(i == nx - 1 && b1 == BC_OUTLET && cx == -1, ic - 1, uo)
-            OUTF(j == 0 && b2 == BC_OUTLET && cy == 1, ic + sy, vo)
-            OUTF(j == ny - 1 && b2 == BC_OUTLET && cy == -1, ic - sy, vo)
-            OUTF(k == 0 && b3 == BC_OUTLET && cz == 1, ic + sz, wo)
-            OUTF(k == nz - 1 && b3 == BC_OUTLET && cz == -1, ic - sz, wo)
-#undef OUTF
-        }
+        if (b1 == BC_OUTLET && (i == 0 || i == nx - 1)) outlet19<0, S>(ft, fs, a.fstride, ic, i == 0, 1, is3 - a.u_o[ic]);
+        if (b2 == BC_OUTLET && (j == 0 || j == ny - 1)) outlet19<1, S>(ft, fs, a.fstride, ic, j == 0, sy, is3 - a.v_o[ic]);
+        if (b3 == BC_OUTLET && (k == 0 || k == nz - 1)) outlet19<2, S>(ft, fs, a.fstride, ic, k == 0, sz, is3 - a.w_o[ic]);
     }
 }
 
