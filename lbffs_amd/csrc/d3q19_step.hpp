@@ -856,11 +856,11 @@ __device__ inline uint32_t face_blocks(const A &a)
 }
 
 // Waves per SIMD the step kernel is held to: eight (64 VGPRs), which the compiler reaches
-// without spilling by interleaving each direction's pull address with its load; seven for
-// the FP32 WALE kernel with interpolated bounce-back, which spills at eight; FP64 as the
-// compiler chooses.
+// without spilling by interleaving each direction's pull address with its load; seven with
+// the interpolated bounce-back, whose groups of links spill at eight; FP64 as the compiler
+// chooses.
 template <typename S, typename Real, int SGS, bool IBB>
-constexpr int kStep19MinWaves = sizeof(Real) == 8 ? 1 : ((IBB && SGS == 0 && sizeof(S) == 4) ? 7 : 8);
+constexpr int kStep19MinWaves = sizeof(Real) == 8 ? 1 : (IBB ? 7 : 8);
 
 template <typename S, typename Real, int SGS, bool IBB = false, int AA = 0, int PASS = 0>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStep19MinWaves<S, Real, SGS, IBB>, 8)))
