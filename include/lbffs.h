@@ -211,10 +211,11 @@ enum {
                                    (from a list) and the others the cells off the faces, so that
                                    no wave runs both paths (two-lattice streaming; takes
                                    precedence over LBFFS_TUNE_SPLIT_FACES) */
-    LBFFS_TUNE_XCD_CHUNK = 64   /* deal runs of 4 consecutive work-groups to each XCD in turn:
+    LBFFS_TUNE_XCD_CHUNK = 64   /* deal runs of 8 consecutive work-groups to each XCD in turn:
                                    the cache line a block shares with its x-neighbour block is
                                    fetched once, not once per XCD (takes precedence over
-                                   LBFFS_TUNE_NO_XCD) */
+                                   LBFFS_TUNE_NO_XCD).  A new context of 262144 cells or more
+                                   starts with it, a smaller one with no option */
 };
 
 /* Autotuner: time every candidate work-group size (64, 128, 256) and launch option on

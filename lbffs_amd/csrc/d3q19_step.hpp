@@ -137,7 +137,11 @@ __device__ inline uint32_t xcd_block(uint32_t pid, uint32_t G)
 // one cache line of its neighbour block; in hardware order that neighbour runs on another
 // XCD and the line is fetched twice (once per L2), in chunks only every C-th block edge
 // crosses XCDs.  The blocks past the last whole group of 8C keep their own number.
-constexpr uint32_t kXcdChunk = 4;
+// Eight blocks (2048 cells: the rows beside a row of a few hundred cells run on the same XCD,
+// which the velocity gradient reads) measured as fast as or faster than 4, 16 and 64:
+// backstep 768x192x128 FP32 466 us per step (4: 474, 16: 464, 64: 470; hardware order 472,
+// slabs 483), D3Q19 WALE channel 160x128x128 85.8 us (87.5, 85.9, 87.1; 88.4, 90.1).
+constexpr uint32_t kXcdChunk = 8;
 __device__ inline uint32_t xcd_chunk_block(uint32_t g, uint32_t G)
 {
     constexpr uint32_t span = 8 * kXcdChunk;

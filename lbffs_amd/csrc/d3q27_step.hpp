@@ -642,14 +642,11 @@ __device__ inline void collide_rr27(Real *ft, Real *K, const Mom19<Real> &m, Rea
     for (int q = 0; q < 27; q++) ft[q] = rho * K[L27::slot[q]] + F * w27<Real>(q) * Real(L27::cx[q]);
 }
 
-// At least seven waves per SIMD (72 VGPRs) for the 32-bit arithmetic: the cumulant update
-// is VALU bound and fits without spilling (eight waves, 64 VGPRs, would spill); the
-// compiler's own choice went as low as five.  FP32 populations with WALE: six (76-78 VGPRs),
-// as the population blocks' pull spills 8 B at seven and the spill-free six ran the bluff
-// body's step in 5.82 against 6.03 ms.  The FP64 form keeps the compiler's choice.
+// Six waves per SIMD (80 VGPRs) for the 32-bit arithmetic: at seven the face path's 27 pulls
+// in flight spill (16-bit forms up to 13 registers), and the BF16 wind tunnel 448x168x140 ran
+// 394 us per step against 367 us at six.  The FP64 form keeps the compiler's choice.
 template <typename S, typename Real, int SGS>
-constexpr int kStep27MinWaves = sizeof(Real) == 8 ? 1 : ((sizeof(S) == 4 && SGS == 0) ? 6 : 7);
-// the batch kernel's extra indirection spills at seven: six
+constexpr int kStep27MinWaves = sizeof(Real) == 8 ? 1 : 6;
 template <typename Real>
 constexpr int kBatch27MinWaves = sizeof(Real) == 8 ? 1 : 6;
 
