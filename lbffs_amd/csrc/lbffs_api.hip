@@ -101,7 +101,9 @@ struct lbffs_ctx {
     void *Gm = nullptr;        // 3n host reals: G_x[n], G_y[n], G_z[n]
     uint32_t *mark = nullptr;  // per-cell stamp of the last spread that touched it
     int *list = nullptr;       // cells touched by the last spread (capacity 8n)
-    int *count = nullptr;
+    int *count = nullptr;      // lengths of the lists of even and odd steps: a step's force kernel
+                               // clears the other, which the last step's list is done with
+    int list_par = 0;          // which of the two the next step's list uses
     uint32_t stamp = 0;
     double motion[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     bool g_dirty = true;       // G may hold values outside the last list
@@ -698,15 +700,15 @@ int ibm_after_step(lbffs_ctx *c, bool last)
     const IbmMotion<Real> m = ibm_motion<Real>(c);
     const int nx = c->d.nx, ny = c->d.ny, nz = c->d.nz;
     c->stamp = (c->stamp == 0xffffffffu) ? 1u : c->stamp + 1u;
-    hipLaunchKernelGGL((ibm_gwall_kernel<Real>), dim3(grid_for(n, 256)), dim3(256), 0, c->stream, n,
-                       (const Real *)c->markers, nx, ny, nz, (const Real *)c->u[c->mcur], (const Real *)c->v[c->mcur],
-                       (const Real *)c->w[c->mcur], m, (Real *)c->Gm, c->count);
-    hipLaunchKernelGGL((ibm_spread_move_kernel<Real>), dim3(grid_for(n, 256)), dim3(256), 0, c->stream, n,
-                       (Real *)c->markers, nx, ny, nz, (const Real *)c->Gm, m, (Real *)c->Gx, (Real *)c->Gy,
-                       (Real *)c->Gz, c->mark, c->stamp, c->list, c->count, cap);
-    hipLaunchKernelGGL((ibm_force_kernel<S, Real, Q>), dim3(grid_for(cap, 256)), dim3(256), 0, c->stream,
-                       (const int *)c->list, (const int *)c->count, cap, c->fstride, (S *)c->f[c->cur], c->flag,
+    int *count = c->count + c->list_par, *next = c->count + (c->list_par ^ 1);
+    hipLaunchKernelGGL((ibm_spread_move_kernel<Real>), dim3(grid_for(n, kIbmBlock)), dim3(kIbmBlock), 0, c->stream, n,
+                       (Real *)c->markers, nx, ny, nz, (const Real *)c->u[c->mcur], (const Real *)c->v[c->mcur],
+                       (const Real *)c->w[c->mcur], m, (Real *)c->Gm, (Real *)c->Gx, (Real *)c->Gy, (Real *)c->Gz,
+                       c->mark, c->stamp, c->list, count, cap);
+    hipLaunchKernelGGL((ibm_force_kernel<S, Real, Q>), dim3(grid_for(cap, kIbmBlock)), dim3(kIbmBlock), 0, c->stream,
+                       (const int *)c->list, (const int *)count, next, cap, c->fstride, (S *)c->f[c->cur], c->flag,
                        (const Real *)c->rho[c->mcur], (Real *)c->Gx, (Real *)c->Gy, (Real *)c->Gz, last ? 0 : 1);
+    c->list_par ^= 1;
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -723,8 +725,8 @@ int ibm_clear_g(lbffs_ctx *c)
     } else {
         const int cap = 8 * c->n_markers;
         hipLaunchKernelGGL((ibm_zero_listed_kernel<Real>), dim3(grid_for(cap, 256)), dim3(256), 0, c->stream,
-                           (const int *)c->list, (const int *)c->count, cap, (Real *)c->Gx, (Real *)c->Gy,
-                           (Real *)c->Gz);
+                           (const int *)c->list, (const int *)(c->count + (c->list_par ^ 1)), cap, (Real *)c->Gx,
+                           (Real *)c->Gy, (Real *)c->Gz);
     }
     HIP_TRY(hipGetLastError());
     return 0;
@@ -1529,11 +1531,12 @@ int lbffs_ibm_set_markers(lbffs_ctx *c, const void *xyz, int n)
     if (!e) e = dalloc(&c->Gm, m3);
     if (!e) e = dalloc((void **)&c->mark, (size_t)c->N * sizeof(uint32_t));
     if (!e) e = dalloc((void **)&c->list, (size_t)8 * n * sizeof(int));
-    if (!e) e = dalloc((void **)&c->count, sizeof(int));
+    if (!e) e = dalloc((void **)&c->count, 2 * sizeof(int));
     if (e) return e;
     HIP_TRY(hipMemcpy(c->markers, xyz, m3, hipMemcpyHostToDevice));
     c->n_markers = n;
     c->stamp = 0;
+    c->list_par = 0;
     c->g_dirty = true;
     return 0;
 }

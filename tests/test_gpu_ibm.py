@@ -102,3 +102,22 @@ def test_one_marker_switches_ibm_off():
     a = run_hip(c, 20)
     b = run_hip(c, 20, ibm={"xyz": np.array([16.0, 12.0, 3.0]), "motion": MOTION})
     assert np.array_equal(a["f"], b["f"])
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 200])
+def test_ibm_scattered_markers(n):
+    """Marker counts around a wave of 64; markers that share cells, that lie in the last layer
+    (some corners of their box outside the lattice) and outside it altogether."""
+    c = _case(19)
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform([1, 1, 1], [c.nx - 2, c.ny - 2, c.nz - 2], size=(n, 3))
+    xyz[0] = [c.nx - 0.5, c.ny - 0.6, c.nz - 0.7]
+    if n > 8:
+        xyz[1:4] = xyz[4] + rng.uniform(0, 0.01, (3, 3))
+        xyz[5], xyz[6], xyz[7] = [-2.5, 4, 4], [c.nx + 3, 5, 5], [10, 10, -0.5]
+    ibm = {"xyz": xyz.astype(np.float32).reshape(-1), "motion": MOTION}
+    h, o32, o64 = parity(c, 6, label=f"ibm scattered {n}", ibm=ibm)
+    assert np.abs(h["ibm_xyz"].astype(np.float64) - o64["ibm_xyz"]).max() <= 1e-4
+    assert rel_l2(h["ibm_G"], o64["ibm_G"]) <= 1e-3
+    G = [np.concatenate([d[g] for g in ("GxIBM", "GyIBM", "GzIBM")]) for d in (h, o64)]
+    assert rel_l2(*G) <= 1e-3
