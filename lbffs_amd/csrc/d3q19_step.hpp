@@ -307,7 +307,34 @@ __device__ inline Real grad_comp(const Real *old, Real self, uint32_t ic, int po
     return lo ? p - self : (hi ? self - m : inside);
 }
 
-// kernel.cl:2267-2365 waleTauSGS (Cw = 0.325) from the velocity gradient
+// x / 3 as the division rounds it: the product with fl(1/3) and one correction by the exact
+// remainder (equal to x / 3.0f for every finite float, checked exhaustively), 3 instructions
+// where the division takes 10.  FP64 divides.
+__device__ inline float div3(float x)
+{
+    const float z = 1.0f / 3.0f;
+    const float q = x * z;
+    return __builtin_fmaf(__builtin_fmaf(-3.0f, q, x), z, q);
+}
+__device__ inline double div3(double x) { return x / 3.0; }
+
+// square root of x in [2^-96, inf], correctly rounded as sqrt() is: the hardware's value is
+// within one ulp, and the signs of the remainders x - (s -+ 1 ulp) s tell which of the three
+// neighbours is nearest.  sqrt() adds the scaling of tiny arguments and the tests for 0, inf
+// and NaN around the same correction, 23 instructions against 8.
+__device__ inline float sqrt_normal(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float dn = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);
+    const float rd = __builtin_fmaf(-dn, s, x), ru = __builtin_fmaf(-up, s, x);
+    const float r = rd <= 0.0f ? dn : s;
+    return ru > 0.0f ? up : r;
+}
+__device__ inline double sqrt_normal(double x) { return sqrt(x); }
+
+// kernel.cl:2267-2365 waleTauSGS (Cw = 0.325) from the velocity gradient.  The D3Q27 step is
+// bound by vector issue and the D3Q19 step near it: hence div3 and sqrt_normal (both sums
+// are above 1e-24 where they are used).
 template <typename Real>
 __device__ inline Real wale_from_grad(Real dudx, Real dudy, Real dudz, Real dvdx, Real dvdy, Real dvdz, Real dwdx,
                                       Real dwdy, Real dwdz)
@@ -326,14 +353,15 @@ __device__ inline Real wale_from_grad(Real dudx, Real dudy, Real dudz, Real dvdx
     Real g31 = dudz * dudx + dvdz * dudy + dwdz * dudz;
     Real g32 = dudz * dvdx + dvdz * dvdy + dwdz * dvdz;
     Real g33 = dudz * dwdx + dvdz * dwdy + dwdz * dwdz;
-    Real tr3 = (g11 + g22 + g33) / Real(3);
+    Real tr3 = div3(g11 + g22 + g33);
     Real d11 = g11 - tr3, d22 = g22 - tr3, d33 = g33 - tr3;
     Real d12 = Real(0.5) * (g12 + g21), d13 = Real(0.5) * (g13 + g31), d23 = Real(0.5) * (g23 + g32);
     Real SdSd = d11 * d11 + d22 * d22 + d33 * d33 + Real(2) * (d12 * d12 + d13 * d13 + d23 * d23);
     if (!(SS > Real(1e-24) && SdSd > Real(1e-24))) return Real(0);
-    Real sd15 = SdSd * sqrt(SdSd);          // SdSd^1.5
-    Real ss25 = SS * SS * sqrt(SS);         // SS^2.5
-    Real sd125 = SdSd * sqrt(sqrt(SdSd));        // SdSd^1.25
+    const Real rSd = sqrt_normal(SdSd);
+    Real sd15 = SdSd * rSd;                 // SdSd^1.5
+    Real ss25 = SS * SS * sqrt_normal(SS);  // SS^2.5
+    Real sd125 = SdSd * sqrt_normal(rSd);   // SdSd^1.25
     return Real(9) * (Cw * Cw * sd15 / (ss25 + sd125));
 }
 
