@@ -4,8 +4,8 @@
  * The reference builds the solid flags and the wall distances on the host before its
  * time loop (D3Q19_opencl/ns.cpp:188-226, the same in D3Q27_opencl/ns.cpp): setSolid
  * from the walls STL, setNeiSolid, setSDF per patch when LES is on, then
- * setSDFnearBwalls.  These entry points replace setSolid and setSDF with HIP kernels;
- * setNeiSolid and setSDFnearBwalls are host functions of lbffs_case.h.
+ * setSDFnearBwalls.  These entry points replace setSolid, setNeiSolid and setSDF with HIP
+ * kernels; setNeiSolid is also a host function of lbffs_case.h, as setSDFnearBwalls is.
  *
  * Triangles come as three (or two) arrays of 3*n floats, one row per axis (x row, then
  * y row, then z row), like STLpatch::STLv0/STLv1/STLv2, STLc and STLnormal
@@ -33,6 +33,11 @@ extern "C" {
  * reference host (FP32, no contraction). */
 int lbffs_geom_solid(int n, const float *v0, const float *v1, const float *v2, int nx, int ny, int nz, int invert,
                      uint8_t *solid);
+
+/* src/walls.hpp:187-216 setNeiSolid on the GPU: lbffs_case_neisolid's flags (lbffs_case.h),
+ * neiSolid = 1 on fluid cells (solid == 0) off the lattice faces with a cell of solid == 1
+ * among their D3Q19 or D3Q27 neighbours, 0 elsewhere.  solid, neiSolid: nx*ny*nz bytes. */
+int lbffs_geom_neisolid(int q, int nx, int ny, int nz, const uint8_t *solid, uint8_t *neiSolid);
 
 /* src/walls.hpp:218-297 setSDF (the per-patch overload called by ns.cpp:205-213).  Every
  * cell within int(dr) cells (a box, clamped to the lattice) of a cell with neiSolid == 1

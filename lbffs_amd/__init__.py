@@ -124,6 +124,7 @@ def lib():
         L.lbffs_batch_destroy.argtypes = [vp]
         fl = C.c_float
         L.lbffs_geom_solid.argtypes = [ip, vp, vp, vp, ip, ip, ip, ip, vp]
+        L.lbffs_geom_neisolid.argtypes = [ip, ip, ip, ip, vp, vp]
         L.lbffs_geom_sdf.argtypes = [ip, vp, vp, fl, fl, fl, ip, ip, ip, vp, vp]
         L.lbffs_geom_qlinks.argtypes = [ip, ip, vp, vp, vp, ip, ip, ip, vp, vp, vp, C.POINTER(ip)]
         L.lbffs_geom_qlinks_ctx.argtypes = [vp, ip, vp, vp, vp, fl, C.POINTER(ip)]
@@ -143,7 +144,7 @@ def lib():
                   "lbffs_autotune", "lbffs_set_launch",
                   "lbffs_ibm_set_markers", "lbffs_ibm_set_motion", "lbffs_ibm_download", "lbffs_batch_create",
                   "lbffs_batch_context", "lbffs_batch_set_launch", "lbffs_batch_step", "lbffs_batch_last_step_ms",
-                  "lbffs_batch_autotune", "lbffs_batch_destroy", "lbffs_geom_solid", "lbffs_geom_sdf",
+                  "lbffs_batch_autotune", "lbffs_batch_destroy", "lbffs_geom_solid", "lbffs_geom_neisolid", "lbffs_geom_sdf",
                   "lbffs_geom_qlinks", "lbffs_geom_qlinks_ctx",
                   "lbffs_case_sdf_near_bwalls",
                   "lbffs_output_macros", "lbffs_out_write_vtk", "lbffs_out_write_restart", "lbffs_out_read_restart",

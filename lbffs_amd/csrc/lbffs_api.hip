@@ -2042,26 +2042,43 @@ int lbffs_geom_solid(int n, const float *v0, const float *v1, const float *v2, i
         box.zmin = fminf(box.zmin, g.zmin);
         box.zmax = fmaxf(box.zmax, g.zmax);
     }
-    // triangles by the z layers their box may cover (a superset: the kernel applies the
-    // exact test of walls.hpp:116-121); a box with a NaN bound covers no layer, as the
-    // reference's comparisons fail for it
-    std::vector<int> bin_start((size_t)nz + 1, 0), bin_tri;
+    // triangles by the z layers and groups of eight rows their box may cover (a superset: the
+    // kernel applies the exact test of walls.hpp:116-121); a box with a NaN bound covers none, as
+    // the reference's comparisons fail for it.  Where large triangles would fill more than 2^26
+    // entries, by layer alone.
+    std::vector<std::array<int, 4>> span((size_t)n, {0, -1, 0, -1});
+    auto cover = [](float lo, float hi, int len, int &first, int &last) {
+        if (!(lo <= hi)) return;
+        const double a = std::max(std::floor((double)lo) - 1.0, 0.0);
+        const double e = std::min(std::ceil((double)hi) + 1.0, (double)(len - 1));
+        if (a > e) return;
+        first = (int)a;
+        last = (int)e;
+    };
+    int jrows = 8;
+    double entries = 0;
+    for (int t = 0; t < n; t++) {
+        cover(tris[t].zmin, tris[t].zmax, nz, span[t][0], span[t][1]);
+        cover(tris[t].ymin, tris[t].ymax, ny, span[t][2], span[t][3]);
+        if (span[t][1] < 0 || span[t][3] < 0) span[t] = {0, -1, 0, -1};
+        else entries += (double)(span[t][1] - span[t][0] + 1) * (span[t][3] / jrows - span[t][2] / jrows + 1);
+    }
+    if (entries > (double)(1 << 26)) jrows = ny;
+    const int jbins = (ny + jrows - 1) / jrows;
+    const size_t nbins = (size_t)jbins * (size_t)nz;
+    std::vector<int> bin_start(nbins + 1, 0), bin_tri;
+    auto each_bin = [&](int t, auto &&f) {
+        for (int k = span[t][0]; k <= span[t][1]; k++)
+            for (int m = span[t][2] / jrows; m <= span[t][3] / jrows; m++) f((size_t)m + (size_t)jbins * (size_t)k);
+    };
+    for (int t = 0; t < n; t++)
+        if (span[t][1] >= 0) each_bin(t, [&](size_t b) { bin_start[b + 1]++; });
+    for (size_t b = 0; b < nbins; b++) bin_start[b + 1] += bin_start[b];
+    bin_tri.resize((size_t)bin_start[nbins]);
     {
-        std::vector<std::pair<int, int>> span((size_t)n, {1, 0});
-        for (int t = 0; t < n; t++) {
-            const float lo = tris[t].zmin, hi = tris[t].zmax;
-            if (!(lo <= hi)) continue;
-            const double klo = std::max(std::floor((double)lo) - 1.0, 0.0);
-            const double khi = std::min(std::ceil((double)hi) + 1.0, (double)(nz - 1));
-            if (klo > khi) continue;
-            span[t] = {(int)klo, (int)khi};
-            for (int k = (int)klo; k <= (int)khi; k++) bin_start[k + 1]++;
-        }
-        for (int k = 0; k < nz; k++) bin_start[k + 1] += bin_start[k];
-        bin_tri.resize((size_t)bin_start[nz]);
         std::vector<int> fill(bin_start.begin(), bin_start.end() - 1);
         for (int t = 0; t < n; t++)
-            for (int k = span[t].first; k <= span[t].second; k++) bin_tri[(size_t)fill[k]++] = t;
+            if (span[t][1] >= 0) each_bin(t, [&](size_t b) { bin_tri[(size_t)fill[b]++] = t; });
     }
     GeomScratch g;
     uint8_t *d_solid;
@@ -2079,13 +2096,31 @@ int lbffs_geom_solid(int n, const float *v0, const float *v1, const float *v2, i
     const size_t blocks = (size_t)chunks * ny * nz;
     if (blocks > 0x7fffffffu) return fail(LBFFS_E_INVALID, "lattice too large for the solid launch");
     hipLaunchKernelGGL(lbffs::geom_solid_kernel, dim3((unsigned)blocks), dim3(lbffs::kGeomRow), 0, nullptr, d_tris,
-                       d_start, d_bins, nx, ny, chunks, box, d_solid);
+                       d_start, d_bins, jrows, jbins, nx, ny, chunks, box, d_solid);
     HIP_TRY(hipGetLastError());
     if (invert) {
         hipLaunchKernelGGL(lbffs::geom_invert_kernel, dim3(geom_grid(N)), dim3(256), 0, nullptr, d_solid, N);
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipMemcpy(solid, d_solid, N, hipMemcpyDeviceToHost));
+    return 0;
+}
+
+int lbffs_geom_neisolid(int q, int nx, int ny, int nz, const uint8_t *solid, uint8_t *neiSolid)
+{
+    if (!solid || !neiSolid) return fail(LBFFS_E_INVALID, "null argument");
+    if (q != 19 && q != 27) return fail(LBFFS_E_INVALID, "q must be 19 or 27");
+    if (int e = geom_dims_ok(nx, ny, nz)) return e;
+    const size_t N = (size_t)nx * ny * nz;
+    GeomScratch g;
+    uint8_t *d_solid, *d_nei;
+    if (int e = g.alloc(&d_solid, N)) return e;
+    if (int e = g.alloc(&d_nei, N)) return e;
+    HIP_TRY(hipMemcpy(d_solid, solid, N, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(lbffs::geom_neisolid_kernel, dim3(geom_grid(N)), dim3(256), 0, nullptr, d_solid, d_nei, q, nx, ny,
+                       nz);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpy(neiSolid, d_nei, N, hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -2152,13 +2187,10 @@ int lbffs_geom_sdf(int n, const float *centroid, const float *normal, float sdf_
     const int drn = (int)dr;
     GeomScratch g;
     uint8_t *d_nei, *d_m1, *d_m2;
-    uint32_t *d_list, *d_count;
     float *d_tri, *d_sdf;
     if (int e = g.alloc(&d_nei, N)) return e;
     if (int e = g.alloc(&d_m1, N)) return e;
     if (int e = g.alloc(&d_m2, N)) return e;
-    if (int e = g.alloc(&d_list, N)) return e;
-    if (int e = g.alloc(&d_count, 1)) return e;
     if (int e = g.alloc(&d_tri, (size_t)6 * n)) return e;
     if (int e = g.alloc(&d_sdf, N)) return e;
     HIP_TRY(hipMemcpy(d_nei, neiSolid, N, hipMemcpyHostToDevice));
@@ -2171,16 +2203,15 @@ int lbffs_geom_sdf(int n, const float *centroid, const float *normal, float sdf_
     hipLaunchKernelGGL(lbffs::geom_dilate_kernel, dim3(gr), dim3(256), 0, nullptr, d_nei, d_m1, nx, ny, nz, 0, drn, 1);
     hipLaunchKernelGGL(lbffs::geom_dilate_kernel, dim3(gr), dim3(256), 0, nullptr, d_m1, d_m2, nx, ny, nz, 1, drn, 0);
     hipLaunchKernelGGL(lbffs::geom_dilate_kernel, dim3(gr), dim3(256), 0, nullptr, d_m2, d_m1, nx, ny, nz, 2, drn, 0);
-    hipLaunchKernelGGL(lbffs::geom_near_list_kernel, dim3(gr), dim3(256), 0, nullptr, d_m1, N, d_list, d_count);
     HIP_TRY(hipGetLastError());
-    uint32_t count = 0;
-    HIP_TRY(hipMemcpy(&count, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (count > N) return fail(LBFFS_E_DEVICE, "near-cell count exceeds the lattice");
-    if (count) {
-        hipLaunchKernelGGL(lbffs::geom_sdf_kernel, dim3((count + 255) / 256), dim3(256), 0, nullptr, d_list, count, d_tri,
-                           n, nx, ny, sdf_ini, dr, p, d_sdf);
-        HIP_TRY(hipGetLastError());
-    }
+    const int bx = (nx + lbffs::kSdfX - 1) / lbffs::kSdfX, by = (ny + lbffs::kSdfY - 1) / lbffs::kSdfY;
+    const size_t blocks = (size_t)bx * by * ((nz + lbffs::kSdfZ - 1) / lbffs::kSdfZ);
+    if (blocks > 0x7fffffffu) return fail(LBFFS_E_INVALID, "lattice too large for the distance launch");
+    const float reach = dr * 1.001f + 0.01f + 1e-6f * (float)std::max(nx, std::max(ny, nz));
+    const int ip = (p >= 1.f && p <= 16.f && p == std::floor(p)) ? (int)p : 0;
+    hipLaunchKernelGGL(lbffs::geom_sdf_kernel, dim3((unsigned)blocks), dim3(lbffs::kSdfBlock), 0, nullptr, d_m1, d_tri, n,
+                       nx, ny, nz, bx, by, sdf_ini, dr, reach, p, ip, d_sdf);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(sdf, d_sdf, N * sizeof(float), hipMemcpyDeviceToHost));
     return 0;
 }

@@ -5,7 +5,7 @@ The sequence is the reference host's (D3Q19_opencl/ns.cpp:188-226, the same in
 D3Q27_opencl/ns.cpp): read the STL scaled by the cell size L (src/stl.hpp:456-557),
 setSolid, setNeiSolid, setSDF for every patch when LES is on (dr 10, p 7, sdfIni 10000),
 then setSDFnearBwalls with dr 3.  setSolid and setSDF run as HIP kernels
-(``include/lbffs_geom.h``); setNeiSolid and setSDFnearBwalls are host functions
+(``include/lbffs_geom.h``), setNeiSolid too; setSDFnearBwalls is a host function
 (``include/lbffs_case.h``).
 """
 from __future__ import annotations
@@ -19,7 +19,6 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import _check, _ptr, lib
-from .cases import neisolid
 
 SDF_INI = 10000.0  # ns.cpp:201
 SDF_DR = 10.0      # ns.cpp:202
@@ -216,6 +215,15 @@ def set_solid(stl: STL, nx: int, ny: int, nz: int, invert: bool = False, solid=N
     return solid_from_triangles(*stl.triangles(), nx, ny, nz, invert, solid)
 
 
+def nei_solid(q: int, nx: int, ny: int, nz: int, solid) -> np.ndarray:
+    """walls.hpp:187-216 setNeiSolid on the GPU (cases.neisolid is the host's)."""
+    s = np.ascontiguousarray(solid, np.uint8)
+    assert s.size == nx * ny * nz
+    out = np.empty_like(s)
+    _check(lib().lbffs_geom_neisolid(q, nx, ny, nz, _ptr(s), _ptr(out)), "lbffs_geom_neisolid")
+    return out
+
+
 def set_sdf(patch: Patch, sdf: np.ndarray, nei: np.ndarray, nx: int, ny: int, nz: int, dr: float = SDF_DR,
             p: float = SDF_P, sdf_ini: float = SDF_INI) -> np.ndarray:
     """walls.hpp:218-297 setSDF (patch form) on the GPU; updates and returns sdf."""
@@ -284,7 +292,7 @@ def sdf_near_bwalls(sdf: np.ndarray, b1, b2, b3, nx: int, ny: int, nz: int, dr: 
 def preprocess(stl: STL, q: int, nx: int, ny: int, nz: int, LES: bool, b1, b2, b3, invert: bool = False) -> dict:
     """ns.cpp:188-226: solid, neiSolid and sdf of a case from its walls STL."""
     solid = set_solid(stl, nx, ny, nz, invert)
-    nei = neisolid(q, nx, ny, nz, solid)
+    nei = nei_solid(q, nx, ny, nz, solid)
     sdf = np.full(nx * ny * nz, SDF_INI, np.float32)
     if LES:
         for p in stl.patches:

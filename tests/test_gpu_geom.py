@@ -221,3 +221,37 @@ def test_qlinks_into_lattice_equal_host_route(storage):
     assert miss == c.meta["qlink_misses"]
     assert np.array_equal(d, host.astype(d.dtype))
     assert (host != 0.5).sum() > 3000
+
+
+@pytest.mark.parametrize("q", [19, 27])
+@pytest.mark.parametrize("dims", [(5, 4, 3), (33, 17, 9), (64, 8, 8), (1, 12, 11), (13, 1, 10), (12, 11, 1), (2, 5, 5)])
+def test_neisolid_equals_host(dims, q):
+    nx, ny, nz = dims
+    solid = (np.random.default_rng(nx * ny + nz).random(nx * ny * nz) < 0.15).astype(np.uint8)
+    assert np.array_equal(geo.nei_solid(q, nx, ny, nz, solid), cases.neisolid(q, nx, ny, nz, solid))
+
+
+@pytest.mark.parametrize("n_lat,n_lon", [(9, 16), (17, 16), (33, 32)])  # 256, 512 and 2048 triangles
+@pytest.mark.parametrize("dims", [(40, 40, 40), (43, 37, 34)])
+def test_sdf_and_solid_box_edges(dims, n_lat, n_lon):
+    """Lattices that are and are not whole 8x8x4 boxes and 8-row bins; triangle counts that fill
+    whole tiles of 256 and, with three triangles left out or one added, do not."""
+    nx, ny, nz = dims
+    body = geo.procedural_body((20.3, 19.1, 18.4), 10.0, n_lat=n_lat, n_lon=n_lon)
+    v = body.triangles()
+    solid = geo.solid_from_triangles(*v, nx, ny, nz)
+    assert np.array_equal(solid, po.geom_solid(*v, nx, ny, nz))
+    nei = cases.neisolid(19, nx, ny, nz, solid)
+    p = body.patches[0]
+    for keep in (p.n, p.n - 3, 1):
+        for power in (7.0, 2.5):
+            cut = geo.Patch("cut", c=np.ascontiguousarray(p.c[:, :keep]), normal=np.ascontiguousarray(p.normal[:, :keep]),
+                            v0=p.v0[:, :keep])
+            start = np.full(nx * ny * nz, 10000.0, np.float32)
+            o = po.geom_sdf(cut.c, cut.normal, start, nei, nx, ny, nz, p=power)
+            g = geo.set_sdf(cut, start.copy(), nei, nx, ny, nz, p=power)
+            # the same terms in the same order: what differs is a weight that the host's powf
+            # rounds the other way (2^-24 of it), on distances of at most 10
+            assert np.array_equal(g == 10000.0, o == 10000.0)
+            assert np.abs(g - o).max() <= 2e-5
+            assert (g == o).mean() > 0.9
