@@ -21,12 +21,15 @@
 #include "ibm.hpp"
 #include "launch.hpp"
 #include "geom.hpp"
+#include "transfer.hpp"
 
 using namespace lbffs;
 
 namespace {
 
 thread_local std::string g_last_error;
+
+HostStage g_stage;  // pinned ring of the large copies, kept while a context lives
 
 int fail(int code, const std::string &msg)
 {
@@ -417,18 +420,25 @@ int scratch_setup(int device)
     return 0;
 }
 
-int dalloc(void **p, size_t bytes)
+// device memory that is written before it is read (no fill)
+int dalloc_raw(void **p, size_t bytes)
 {
-    hipError_t e = hipMalloc(p, bytes);
+    const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
         return fail(LBFFS_E_NOMEM, std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
     }
+    return 0;
+}
+
+int dalloc(void **p, size_t bytes)
+{
+    if (int r = dalloc_raw(p, bytes)) return r;
     // hipMemset runs on the null stream and may return before it has finished; the
     // contexts' streams are non-blocking and do not wait for it, so a kernel that writes
     // the new buffer right away (the decode of a 16-bit download, for one) could be
     // overwritten by the zeros: wait for the fill here.
-    e = hipMemset(*p, 0, bytes);
+    hipError_t e = hipMemset(*p, 0, bytes);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return fail(LBFFS_E_DEVICE, std::string("hipMemset: ") + hipGetErrorString(e));
     return 0;
@@ -521,7 +531,7 @@ int pack_flags(lbffs_ctx *c)
     // the face pass's list: the non-solid lattice-face cells, in index order
     {
         std::vector<uint16_t> fl((size_t)c->N);
-        HIP_TRY(hipMemcpy(fl.data(), c->flag, (size_t)c->N * sizeof(uint16_t), hipMemcpyDeviceToHost));
+        HIP_TRY(g_stage.copy(fl.data(), c->flag, (size_t)c->N * sizeof(uint16_t), hipMemcpyDeviceToHost, c->stream));
         std::vector<uint32_t> cells;
         for (long ic = 0; ic < c->N; ic++)
             if ((fl[ic] & F_FACE) && !(fl[ic] & F_SOLID)) cells.push_back((uint32_t)ic);
@@ -795,8 +805,8 @@ int upload_f(lbffs_ctx *c, const void *host)
     // layout (encode_kernel)
     const size_t n = (size_t)c->d.q * c->N;
     void *tmp = nullptr;
-    if (int e = dalloc(&tmp, n * sizeof(Real))) return e;
-    hipError_t e1 = hipMemcpy(tmp, host, n * sizeof(Real), hipMemcpyHostToDevice);
+    if (int e = dalloc_raw(&tmp, n * sizeof(Real))) return e;
+    hipError_t e1 = g_stage.copy(tmp, host, n * sizeof(Real), hipMemcpyHostToDevice, c->stream);
     if (e1 == hipSuccess) {
         for (int b = 0; b < 2; b++) {
             if (!c->f[b]) continue;
@@ -822,7 +832,7 @@ int download_f(lbffs_ctx *c, void *host)
     const size_t n = (size_t)c->d.q * c->N;
     HIP_TRY(hipStreamSynchronize(c->stream));
     void *tmp = nullptr;
-    if (int e = dalloc(&tmp, n * sizeof(Real))) return e;
+    if (int e = dalloc_raw(&tmp, n * sizeof(Real))) return e;
     if (c->d.q == 27)
         hipLaunchKernelGGL((decode_kernel<S, Real, 27>), dim3(grid_for(c->N, 256)), dim3(256), 0, c->stream,
                            (uint32_t)c->N, c->fstride, (const S *)c->f[c->cur], (Real *)tmp);
@@ -830,8 +840,7 @@ int download_f(lbffs_ctx *c, void *host)
         hipLaunchKernelGGL((decode_kernel<S, Real, 19>), dim3(grid_for(c->N, 256)), dim3(256), 0, c->stream,
                            (uint32_t)c->N, c->fstride, (const S *)c->f[c->cur], (Real *)tmp);
     hipError_t e1 = hipGetLastError();
-    if (e1 == hipSuccess) e1 = hipStreamSynchronize(c->stream);
-    if (e1 == hipSuccess) e1 = hipMemcpy(host, tmp, n * sizeof(Real), hipMemcpyDeviceToHost);
+    if (e1 == hipSuccess) e1 = g_stage.copy(host, tmp, n * sizeof(Real), hipMemcpyDeviceToHost, c->stream);
     hipFree(tmp);
     if (e1 != hipSuccess) return fail(LBFFS_E_DEVICE, std::string("download f: ") + hipGetErrorString(e1));
     return 0;
@@ -894,7 +903,7 @@ int output_macros_impl(lbffs_ctx *c, double dpdx, void *const *host)
 {
     const size_t n = (size_t)c->N;
     void *tmp = nullptr;
-    if (int e = dalloc(&tmp, 4 * n * sizeof(Real))) return e;
+    if (int e = dalloc_raw(&tmp, 4 * n * sizeof(Real))) return e;
     Real *t = (Real *)tmp;
     if (c->d.q == 27)
         hipLaunchKernelGGL((output_macros_kernel<S, Real, 27>), dim3(grid_for(c->N, 256)), dim3(256), 0, c->stream,
@@ -905,8 +914,8 @@ int output_macros_impl(lbffs_ctx *c, double dpdx, void *const *host)
                            (uint32_t)c->N, c->fstride, (const S *)c->f[c->cur], (Real)dpdx, t, t + n, t + 2 * n,
                            t + 3 * n);
     hipError_t e1 = hipGetLastError();
-    if (e1 == hipSuccess) e1 = hipStreamSynchronize(c->stream);
-    for (int a = 0; a < 4 && e1 == hipSuccess; a++) e1 = hipMemcpy(host[a], t + a * n, n * sizeof(Real), hipMemcpyDeviceToHost);
+    for (int a = 0; a < 4 && e1 == hipSuccess; a++)
+        e1 = g_stage.copy(host[a], t + a * n, n * sizeof(Real), hipMemcpyDeviceToHost, c->stream);
     hipFree(tmp);
     if (e1 != hipSuccess) return fail(LBFFS_E_DEVICE, std::string("output macros: ") + hipGetErrorString(e1));
     return 0;
@@ -1154,6 +1163,7 @@ void batch_free(lbffs_batch *b)
     for (lbffs_ctx *c : b->ctx) {
         free_all(c);
         delete c;
+        g_stage.release();
     }
     for (void *p : {b->args_dev[0], b->args_dev[1], b->args_dev[2], b->args_dev[3], (void *)b->table,
                     (void *)b->ftable, (void *)b->fcells, (void *)b->ctr})
@@ -1336,6 +1346,7 @@ int lbffs_create(const lbffs_desc *desc, lbffs_ctx **out)
         delete c;
         return fail(LBFFS_E_DEVICE, std::string("create: ") + hipGetErrorString(he));
     }
+    g_stage.retain();
     *out = c;
     return 0;
 }
@@ -1356,7 +1367,7 @@ int lbffs_upload(lbffs_ctx *c, int field, const void *host, size_t bytes)
     if (field == LBFFS_FIELD_QLINK && !c->qlink) {
         if (int e = dalloc(&c->qlink, bytes)) return e;
     }
-    HIP_TRY(hipMemcpy(field_ptr(c, field), host, bytes, hipMemcpyHostToDevice));
+    HIP_TRY(g_stage.copy(field_ptr(c, field), host, bytes, hipMemcpyHostToDevice, c->stream));
     if (field_affects_flags(field)) c->flags_dirty = true;
     if (field == LBFFS_FIELD_GX || field == LBFFS_FIELD_GY || field == LBFFS_FIELD_GZ) c->g_dirty = true;
     return 0;
@@ -1579,8 +1590,7 @@ int lbffs_download(lbffs_ctx *c, int field, void *host, size_t bytes)
         if (int e = aa_restore(c)) return e;
         return dispatch<DownloadFOp>(c, host);
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipMemcpy(host, field_ptr(c, field), bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(g_stage.copy(host, field_ptr(c, field), bytes, hipMemcpyDeviceToHost, c->stream));
     return 0;
 }
 
@@ -1653,6 +1663,7 @@ int lbffs_destroy(lbffs_ctx *c)
     hipStreamSynchronize(c->stream);
     free_all(c);
     delete c;
+    g_stage.release();
     return 0;
 }
 
@@ -2088,7 +2099,7 @@ int lbffs_geom_solid(int n, const float *v0, const float *v1, const float *v2, i
     if (int e = g.alloc(&d_tris, tris.size())) return e;
     if (int e = g.alloc(&d_start, bin_start.size())) return e;
     if (int e = g.alloc(&d_bins, bin_tri.size())) return e;
-    HIP_TRY(hipMemcpy(d_solid, solid, N, hipMemcpyHostToDevice));
+    HIP_TRY(g_stage.copy(d_solid, solid, N, hipMemcpyHostToDevice, nullptr));
     if (n) HIP_TRY(hipMemcpy(d_tris, tris.data(), tris.size() * sizeof(lbffs::GeomTri), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(d_start, bin_start.data(), bin_start.size() * sizeof(int), hipMemcpyHostToDevice));
     if (!bin_tri.empty()) HIP_TRY(hipMemcpy(d_bins, bin_tri.data(), bin_tri.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -2102,7 +2113,7 @@ int lbffs_geom_solid(int n, const float *v0, const float *v1, const float *v2, i
         hipLaunchKernelGGL(lbffs::geom_invert_kernel, dim3(geom_grid(N)), dim3(256), 0, nullptr, d_solid, N);
         HIP_TRY(hipGetLastError());
     }
-    HIP_TRY(hipMemcpy(solid, d_solid, N, hipMemcpyDeviceToHost));
+    HIP_TRY(g_stage.copy(solid, d_solid, N, hipMemcpyDeviceToHost, nullptr));
     return 0;
 }
 
@@ -2116,11 +2127,11 @@ int lbffs_geom_neisolid(int q, int nx, int ny, int nz, const uint8_t *solid, uin
     uint8_t *d_solid, *d_nei;
     if (int e = g.alloc(&d_solid, N)) return e;
     if (int e = g.alloc(&d_nei, N)) return e;
-    HIP_TRY(hipMemcpy(d_solid, solid, N, hipMemcpyHostToDevice));
+    HIP_TRY(g_stage.copy(d_solid, solid, N, hipMemcpyHostToDevice, nullptr));
     hipLaunchKernelGGL(lbffs::geom_neisolid_kernel, dim3(geom_grid(N)), dim3(256), 0, nullptr, d_solid, d_nei, q, nx, ny,
                        nz);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpy(neiSolid, d_nei, N, hipMemcpyDeviceToHost));
+    HIP_TRY(g_stage.copy(neiSolid, d_nei, N, hipMemcpyDeviceToHost, nullptr));
     return 0;
 }
 
@@ -2141,10 +2152,10 @@ int lbffs_geom_qlinks(int q, int n, const float *v0, const float *v1, const floa
     float *d_q;
     if (int e = g.alloc(&d_solid, N)) return e;
     if (int e = g.alloc(&d_q, (size_t)q * N)) return e;
-    HIP_TRY(hipMemcpy(d_solid, solid, N, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d_q, qlink, (size_t)q * N * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(g_stage.copy(d_solid, solid, N, hipMemcpyHostToDevice, nullptr));
+    HIP_TRY(g_stage.copy(d_q, qlink, (size_t)q * N * sizeof(float), hipMemcpyHostToDevice, nullptr));
     if (int e = qlink_cast(q, surf, nx, ny, nz, cells, d_solid, d_q, nullptr, misses)) return e;
-    HIP_TRY(hipMemcpy(qlink, d_q, (size_t)q * N * sizeof(float), hipMemcpyDeviceToHost));
+    HIP_TRY(g_stage.copy(qlink, d_q, (size_t)q * N * sizeof(float), hipMemcpyDeviceToHost, nullptr));
     return 0;
 }
 
@@ -2193,8 +2204,8 @@ int lbffs_geom_sdf(int n, const float *centroid, const float *normal, float sdf_
     if (int e = g.alloc(&d_m2, N)) return e;
     if (int e = g.alloc(&d_tri, (size_t)6 * n)) return e;
     if (int e = g.alloc(&d_sdf, N)) return e;
-    HIP_TRY(hipMemcpy(d_nei, neiSolid, N, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d_sdf, sdf, N * sizeof(float), hipMemcpyHostToDevice));
+    HIP_TRY(g_stage.copy(d_nei, neiSolid, N, hipMemcpyHostToDevice, nullptr));
+    HIP_TRY(g_stage.copy(d_sdf, sdf, N * sizeof(float), hipMemcpyHostToDevice, nullptr));
     if (n) {
         HIP_TRY(hipMemcpy(d_tri, centroid, (size_t)3 * n * sizeof(float), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(d_tri + (size_t)3 * n, normal, (size_t)3 * n * sizeof(float), hipMemcpyHostToDevice));
@@ -2212,7 +2223,7 @@ int lbffs_geom_sdf(int n, const float *centroid, const float *normal, float sdf_
     hipLaunchKernelGGL(lbffs::geom_sdf_kernel, dim3((unsigned)blocks), dim3(lbffs::kSdfBlock), 0, nullptr, d_m1, d_tri, n,
                        nx, ny, nz, bx, by, sdf_ini, dr, reach, p, ip, d_sdf);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpy(sdf, d_sdf, N * sizeof(float), hipMemcpyDeviceToHost));
+    HIP_TRY(g_stage.copy(sdf, d_sdf, N * sizeof(float), hipMemcpyDeviceToHost, nullptr));
     return 0;
 }
 
