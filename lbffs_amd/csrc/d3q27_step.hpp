@@ -297,6 +297,58 @@ __device__ __forceinline__ void face_cell27(const StepArgs<Real, 27> &a, Real *f
     }
 }
 
+// The face conditions of a cell on an x face and no other (an XMIX wave's), its directions pulled
+// from the interior offsets already, for the codes of x_face_usual: the nine directions that
+// cross the face take one source each -- the cell's own reversed slot across a wall, the far
+// end of the row across a periodic face, the inner neighbour at an outlet, with the cell's own
+// value beside it -- and the velocity or the outlet's rate is loaded with them.  The formulas
+// are face_cell27's.  A wave that ran the interior pull and then the general face path for its
+// one or two x-face cells took half as long again as an interior wave: 257x97x81 FP32 100.5 ->
+// 96 us per step, 240x96x80 FP64 233 -> 191 us (with three waves per SIMD).  Not used for 16-bit
+// values, which are bound by instruction issue either way (448x168x140 BF16: 352 against 355 us).
+template <typename S, typename Real>
+__device__ __forceinline__ void x_face27(const StepArgs<Real, 27> &a, Real *ft, uint32_t fl, uint32_t ic, int i)
+{
+    const int b1 = flag_code(fl, F_B1_SHIFT);
+    const bool fixed = b1 == BC_FIXEDVELOCITY, out = b1 == BC_OUTLET, wall = fixed || b1 == BC_BOUNCEBACK;
+    const S *fs = (const S *)a.fsrc;
+    const bool lo = (i == 0), any_out = __ballot(out) != 0;
+    const Real u = fixed ? a.u0[ic] : a.u_o[ic];
+    const uint32_t inner = lo ? ic + 1u : ic - 1u;
+    S ra[27], rb[27];
+#pragma unroll
+    for (int q = 1; q < 27; q++) {
+        if (L27::cx[q] != 1) continue;
+        const int qo = L27::opp(q);
+        const uint32_t wrap = ic - (uint32_t)(lo ? a.off[q] : a.off[qo]) + (uint32_t)(lo ? a.nx : -a.nx);
+        const uint32_t src = wall ? ic : (out ? inner : wrap);
+        ra[q] = fs[pop_at<27, S>(lo == wall ? qo : q, src, a.fstride)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (any_out) {
+#pragma unroll
+        for (int q = 1; q < 27; q++) {
+            if (L27::cx[q] != 1) continue;
+            rb[q] = fs[pop_at<27, S>(lo ? q : L27::opp(q), ic, a.fstride)];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    const Real s = Real(0.57735026918962576) - u;
+#pragma unroll
+    for (int q = 1; q < 27; q++) {
+        if (L27::cx[q] != 1) continue;
+        const int qo = L27::opp(q);
+        Real v = Codec<S, Real, 27>::load(&ra[q], q, w27<Real>(q));
+        if (any_out) {
+            const Real vo = s * v + (Real(1) - s) * Codec<S, Real, 27>::load(&rb[q], q, w27<Real>(q));
+            v = pick(out, vo, v);
+        }
+        ft[q] = pick(lo, v, ft[q]);
+        ft[qo] = pick(lo, ft[qo], v);
+    }
+    if (fixed) fixed_velocity27<0, S>(a, ft, (long)ic, i, 1, u, a.v0[ic], a.w0[ic]);
+}
+
 // First pass of the moment transform: the populations in slot order (9 z lines of 3),
 // each line reduced to its raw z moments (sum f, sum z f, sum z^2 f).  Density, z momentum
 // and the raw second moments follow from the nine lines with a few additions, so the
@@ -644,11 +696,12 @@ __device__ inline void collide_rr27(Real *ft, Real *K, const Mom19<Real> &m, Rea
 
 // Six waves per SIMD (80 VGPRs) for the 32-bit arithmetic: at seven the face path's 27 pulls
 // in flight spill (16-bit forms up to 13 registers), and the BF16 wind tunnel 448x168x140 ran
-// 394 us per step against 367 us at six.  The FP64 form keeps the compiler's choice.
+// 394 us per step against 367 us at six.  FP64 three, as without those pulls the compiler chose.
 template <typename S, typename Real, int SGS>
-constexpr int kStep27MinWaves = sizeof(Real) == 8 ? 1 : 6;
+constexpr int kStep27MinWaves = sizeof(Real) == 8 ? 3 : 6;
+// FP64 at three runs a batch of 40^3 cavities in 167 against 216 us at two, spills and all
 template <typename Real>
-constexpr int kBatch27MinWaves = sizeof(Real) == 8 ? 1 : 6;
+constexpr int kBatch27MinWaves = sizeof(Real) == 8 ? 3 : 6;
 
 // PASS as step19_kernel: 1 the cells off the lattice faces, 2 the listed face cells, 3 both
 // in one grid (the face-list work-groups first)
@@ -674,8 +727,7 @@ step27_kernel(const StepArgs<Real, 27> a)
 #define CELL_RETURN return
 #define CELL_WALE_INTERIOR true
 #define CELL_SKIP_FACE (PASS == 1 || (PASS == 3 && !face_wg))
-// (the 16-bit split interior pass would spill with the per-wave fast path)
-#define CELL_PURE_OK (!face_wg && !(PASS == 1 && sizeof(S) == 2))
+#define CELL_PURE_OK (!face_wg)
 #define CELL_ALIGNED (!face_wg && a.wave_runs)
 #define CELL_COLL COLL
 #include "d3q27_cell.inc"

@@ -445,9 +445,11 @@ int dalloc(void **p, size_t bytes)
 }
 
 // The class of the run of 64 cells from `first` (wave_class): PURE if all are fluid and off
-// the lattice faces (PLAIN if besides every flag word is zero); on D3Q19 also XMIX if all are
-// fluid and the face cells among them lie on an x face with j and k interior (so that every
-// cell's interior-offset pulls stay in the lattice), or WRAP if all are fluid cells of one row
+// the lattice faces (PLAIN if besides every flag word is zero); XMIX if all are fluid and the
+// face cells among them lie on an x face with j and k interior, so that every cell's
+// interior-offset pulls stay in the lattice (D3Q27: 32- and 64-bit values, with the usual
+// codes, and but for the two cells whose diagonal pull does not); on D3Q19 also WRAP if all are
+// fluid cells of one row
 // with i interior, on a y face and/or a z face whose code is Cyclic for every cell (their
 // pulls wrap like interior pulls shifted by whole rows or planes, and no face condition
 // applies); GENERAL otherwise.
@@ -461,8 +463,11 @@ uint32_t wave_class_of(const lbffs_ctx *c, const uint16_t *fl, size_t first)
         plain = plain && fl[first + l] == 0;
     }
     if (!face) return plain ? WAVE_PLAIN : WAVE_PURE;
-    if (c->d.q != 19) return WAVE_GENERAL;
-    bool xmix = nz >= 3, wrap = true;
+    const bool q27 = c->d.q == 27;
+    // the farthest interior offset: D3Q27's diagonal, which from the lattice's first and last
+    // cells off the y and z faces reaches one cell past the lattice
+    const long far = 1 + (long)nx + (long)nx * ny;
+    bool xmix = nz >= 3 && !(q27 && c->store_size == 2), wrap = !q27;
     const size_t i0 = first % (size_t)nx, r0 = first / (size_t)nx;
     for (size_t l = 0; l < 64; l++) {
         const size_t ic = first + l;
@@ -472,6 +477,7 @@ uint32_t wave_class_of(const lbffs_ctx *c, const uint16_t *fl, size_t first)
         if (f & F_FACE) {
             const bool xonly = (i == 0 || i == nx - 1) && j >= 1 && j <= ny - 2 && k >= 1 && k <= nz - 2;
             xmix = xmix && xonly;
+            if (q27) xmix = xmix && x_face_usual(f) && (long)ic >= far && (long)ic + far < c->N;
         }
         // WRAP: one row, i interior, every face it lies on periodic
         const bool same_row = ic / (size_t)nx == r0 && (l > 0 || i0 == (size_t)i);
@@ -1283,10 +1289,9 @@ int lbffs_create(const lbffs_desc *desc, lbffs_ctx **out)
     c->d = *desc;
     c->device = device;
     c->N = N;
-    // work-groups of 256, 128 for the D3Q27 16-bit forms (448x168x140 BF16: 350 against 361 us
-    // per step; FP32 is indifferent)
-    c->block = desc->block > 0 ? desc->block
-                               : ((desc->q == 27 && desc->storage != LBFFS_STORE_F32 && desc->storage != LBFFS_STORE_F64) ? 128 : 256);
+    // work-groups of 256, 128 for D3Q27 with 32-bit arithmetic (448x168x140 BF16: 350 against
+    // 361 us per step, 257x97x81 FP32 96.1 against 98.1)
+    c->block = desc->block > 0 ? desc->block : ((desc->q == 27 && desc->storage != LBFFS_STORE_F64) ? 128 : 256);
     // Work-groups in XCD chunks where every XCD gets several (1024 blocks of 256 cells): one
     // front through the arrays against eight slabs, D3Q27 257x97x81 FP32 100 against 118 us per
     // step, 448x168x140 BF16 367 against 394, the D3Q19 lattices of xcd_chunk_block's comment

@@ -38,7 +38,8 @@ __host__ __device__ inline int flag_code(uint32_t fl, int shift) { return (int)(
 //   WAVE_PURE     64 fluid cells off the lattice faces: fixed interior offsets;
 //   WAVE_XMIX     64 fluid cells whose face cells lie on an x face only (their j and k
 //                 interior): every cell pulls from the interior offsets (in bounds), then the
-//                 face cells redo the directions that cross their face and apply its conditions;
+//                 face cells redo the directions that cross their face and apply its conditions
+//                 (D3Q27: codes of x_face_usual only);
 //   WAVE_WRAP     64 fluid cells of one row, none on an x face, inside a y and/or z face plane
 //                 whose code is Cyclic for all of them: interior offsets with a periodic wrap
 //                 uniform over the wave;
@@ -68,6 +69,15 @@ __device__ inline uint32_t cell_wave_class(const uint32_t *bits, uint32_t ic)
 // BC codes (input.hpp:221-256)
 enum { BC_CYCLIC = 0, BC_BOUNCEBACK = 1, BC_OUTLET = 3, BC_SYMMETRY = 4, BC_FIXEDVELOCITY = 5,
        BC_FIXEDDENSITY = 6, BC_WALLFUNCTION = 7 };
+
+// a cell on an x face and no other whose flags ask for nothing beyond a wall, a periodic face, a
+// fixed velocity or an outlet, without Symmetry's mirroring (D3Q27's XMIX waves)
+__host__ __device__ inline bool x_face_usual(uint32_t fl)
+{
+    const int b1 = flag_code(fl, F_B1_SHIFT);
+    return (b1 == BC_CYCLIC || b1 == BC_BOUNCEBACK || b1 == BC_OUTLET || b1 == BC_FIXEDVELOCITY) &&
+           flag_code(fl, F_B2_SHIFT) != BC_SYMMETRY && flag_code(fl, F_B3_SHIFT) != BC_SYMMETRY;
+}
 
 // collision operators (the values of LBFFS_COLL_* in lbffs.h)
 enum { COLL_RR = 0, COLL_CUMULANT = 1 };
