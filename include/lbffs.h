@@ -196,7 +196,8 @@ int lbffs_output_macros(lbffs_ctx *ctx, float dpdx, void *rho, void *u, void *v,
 /* Launch options of the step (no counterpart in the reference, whose work-group size
  * is left to the OpenCL runtime, ns.cpp:516). */
 enum {
-    LBFFS_TUNE_NT_STORE = 1, /* accepted, no effect: new populations are always stored non-temporally */
+    LBFFS_TUNE_NT_STORE = 1, /* store the new populations non-temporally also where the 256 MB cache
+                                would hold the step (larger lattices always do) */
     LBFFS_TUNE_NO_XCD = 2,   /* keep the hardware work-group order across the 8 XCDs */
     LBFFS_TUNE_YTILE = 4,    /* visit the cells in tiles of 32, 16 or 8 rows (the first that
                                 divides ny), plane by plane: the neighbour planes WALE reads
@@ -215,7 +216,8 @@ enum {
                                    the cache line a block shares with its x-neighbour block is
                                    fetched once, not once per XCD (takes precedence over
                                    LBFFS_TUNE_NO_XCD).  A new context of 262144 cells or more
-                                   starts with it, a smaller one with no option */
+                                   whose step exceeds the 256 MB cache starts with it, a smaller
+                                   one with no option */
 };
 
 /* Autotuner: time every candidate work-group size (64, 128, 256) and launch option on

@@ -95,6 +95,7 @@ __attribute__((amdgpu_waves_per_eu(Q == 27 ? kBatch27MinWaves<Real> : kBatch19Mi
 #define CELL_SKIP_FACE (PASS == 1)
 #define CELL_PURE_OK (PASS == 1)
 #define CELL_ALIGNED (PASS == 1)
+#define CELL_KEEP false
 #define CELL_COLL COLL
             if constexpr (Q == 27) {
 #include "d3q27_cell.inc"
@@ -102,6 +103,7 @@ __attribute__((amdgpu_waves_per_eu(Q == 27 ? kBatch27MinWaves<Real> : kBatch19Mi
 #include "d3q19_cell.inc"
             }
 #undef CELL_COLL
+#undef CELL_KEEP
 #undef CELL_ALIGNED
 #undef CELL_PURE_OK
 #undef CELL_SKIP_FACE

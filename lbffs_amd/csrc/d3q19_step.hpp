@@ -48,6 +48,7 @@ template <typename Real, int Q>
 struct StepArgs {
     uint32_t N;
     uint32_t fstride;  // 16-bit values: elements between two direction arrays (pop_at)
+    int keep;          // 1: the new populations stay in the caches (fits_cache)
     int wave_runs;     // 1: a wave of the cell order holds one aligned run of 64 cells
     int nx, ny, nz;
     FastDiv dnx, dny;
@@ -87,7 +88,7 @@ using Step19Args = StepArgs<Real, 19>;
 
 // launch options (uniform per launch)
 enum : int {
-    TUNE_NT_STORE = 1,  // accepted, no effect: the populations are always stored non-temporally
+    TUNE_NT_STORE = 1,  // the populations are stored non-temporally whatever the lattice's size (keep)
     TUNE_NO_XCD = 2,    // keep the hardware work-group order (no XCD slab remap)
     TUNE_YTILE = 4,     // visit the cells in y-tiles (see ytile_cell)
     TUNE_SPLIT = 8,     // two passes per step: the cells off the faces, then the face cells
@@ -971,7 +972,9 @@ step19_kernel(const Step19Args<Real> a)
 #define CELL_SKIP_FACE (PASS == 1 || (PASS == 3 && !face_wg))
 #define CELL_PURE_OK (AA == 0 && !face_wg)
 #define CELL_ALIGNED (!face_wg && a.wave_runs)
+#define CELL_KEEP a.keep
 #include "d3q19_cell.inc"
+#undef CELL_KEEP
 #undef CELL_ALIGNED
 #undef CELL_PURE_OK
 #undef CELL_SKIP_FACE

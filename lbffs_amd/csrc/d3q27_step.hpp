@@ -729,9 +729,11 @@ step27_kernel(const StepArgs<Real, 27> a)
 #define CELL_SKIP_FACE (PASS == 1 || (PASS == 3 && !face_wg))
 #define CELL_PURE_OK (!face_wg)
 #define CELL_ALIGNED (!face_wg && a.wave_runs)
+#define CELL_KEEP a.keep
 #define CELL_COLL COLL
 #include "d3q27_cell.inc"
 #undef CELL_COLL
+#undef CELL_KEEP
 #undef CELL_ALIGNED
 #undef CELL_PURE_OK
 #undef CELL_SKIP_FACE

@@ -575,6 +575,21 @@ uint32_t ytile_rows(const lbffs_ctx *c)
     return 0;
 }
 
+// What a two-lattice step reads and writes (two population arrays, two sets of moments, the
+// flags) fits the 256 MB Infinity Cache and is not small: the new populations are then stored so
+// that the next step finds them there, where larger lattices stream them past the caches, whose
+// lines they would only take from the pulls' and the velocity stencil's neighbours.  128x148x69
+// FP32 (240 MB): 44.9 -> 38.5 us per step, 144x158x75 FP16 46.4 -> 38.5, 96x126x54 FP64 47.6 ->
+// 42.8, D3Q27 112x135x61 FP16 37.6 -> 31.7; a fifth larger the streamed form is level or ahead
+// (144x150x73 FP32 55.4 against 56.2, 160x191x86 FP16 66.4 against 70.4).  Below 80 MB the write-back
+// of the L2s at the end of every launch takes back what the hits give (64x72x34 FP32 11.0
+// streamed, 11.6 kept; D3Q27 80x84x41 FP32 17.6 and 18.4).
+bool fits_cache(const lbffs_ctx *c)
+{
+    const double bytes = (double)c->N * (2.0 * c->d.q * c->store_size + 8.0 * c->real_size + 2.0);
+    return c->d.streaming != LBFFS_STREAM_AA && bytes >= 80e6 && bytes <= 256.0 * (1 << 20);
+}
+
 // whether the step kernels of this lattice read its per-wave flag summary: the summary
 // names aligned runs of 64 cells, which a wave covers when its cells are consecutive (the
 // plain order, or y-tiles whose rows are whole waves); off with TUNE_NO_PURE and in-place
@@ -604,6 +619,7 @@ void set_args(lbffs_ctx *c, StepArgs<Real, Q> &a, const lbffs_step_params *p)
         a.off[q] = cx + nx * cy + nx * ny * zoff;
     }
     a.fstride = (uint32_t)c->fstride;
+    a.keep = (fits_cache(c) && !(c->tune & TUNE_NT_STORE)) ? 1 : 0;
     a.flag = c->flag;
     a.u0 = (const Real *)c->u0;
     a.v0 = (const Real *)c->v0;
@@ -1296,9 +1312,11 @@ int lbffs_create(const lbffs_desc *desc, lbffs_ctx **out)
     // front through the arrays against eight slabs, D3Q27 257x97x81 FP32 100 against 118 us per
     // step, 448x168x140 BF16 367 against 394, the D3Q19 lattices of xcd_chunk_block's comment
     // 3-5 %.  Smaller lattices stay in the caches and keep slabs (32^3: 9.9 against 10.4 us).
-    c->tune = N >= 1024 * 256 ? TUNE_XCD_CHUNK : 0;
+    // So do those whose step the Infinity Cache holds: a slab's rows and planes are then written
+    // and read by one XCD (128x148x69 FP32 38.5 against 42.6 us).
     c->real_size = (desc->storage == LBFFS_STORE_F64) ? 8 : 4;
     c->store_size = (desc->storage == LBFFS_STORE_F64) ? 8 : (desc->storage == LBFFS_STORE_F32 ? 4 : 2);
+    c->tune = (N >= 1024 * 256 && !fits_cache(c)) ? TUNE_XCD_CHUNK : 0;
     const size_t n = (size_t)N, rs = c->real_size;
     int e = 0;
     hipError_t he = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);

@@ -289,9 +289,19 @@ __device__ inline uint32_t sr_step(uint32_t step, const uint32_t *ctr)
 // the 19 (27) rounding thresholds of a cell evenly over [0, 1) -- one add per direction
 __device__ inline uint32_t sr_bits(uint32_t h, int q) { return h + (uint32_t)q * 0x9E3779B9u; }
 
+// one value stored, NT: non-temporally
+template <bool NT, typename T>
+__device__ inline void put(T *p, T v)
+{
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
 // Store<S,Real>: load/store of population q with weight w as compute type Real;
-// store_nt_sr(..., r) is the non-temporal store with stochastic rounding from the random
-// bits r (the 32-bit forms store exactly and ignore r).
+// out_sr(..., r) is the store with stochastic rounding from the random
+// bits r (the 32-bit forms store exactly and ignore r); out and out_sr are non-temporal with NT.
 template <typename S, typename Real, int Q>
 struct Codec;
 
@@ -300,13 +310,22 @@ struct Codec<float, float, Q> {
     __device__ static inline float load(const float *p, int, float) { return *p; }
     __device__ static inline float load_nt(const float *p, int, float) { return __builtin_nontemporal_load(p); }
     __device__ static inline void store(float *p, float v, int, float) { *p = v; }
-    __device__ static inline void store_nt(float *p, float v, int, float) { __builtin_nontemporal_store(v, p); }
-    __device__ static inline void store_nt_sr(float *p, float v, int q, float w, uint32_t) { store_nt(p, v, q, w); }
-    __device__ static inline void store_nt_sr2(float *p0, float *p1, float v0, float v1, int q0, int q1, float w0,
-                                               float w1, uint32_t, uint32_t)
+    template <bool NT>
+    __device__ static inline void out(float *p, float v, int, float)
     {
-        store_nt(p0, v0, q0, w0);
-        store_nt(p1, v1, q1, w1);
+        put<NT>(p, v);
+    }
+    template <bool NT>
+    __device__ static inline void out_sr(float *p, float v, int q, float w, uint32_t)
+    {
+        put<NT>(p, v);
+    }
+    template <bool NT>
+    __device__ static inline void out_sr2(float *p0, float *p1, float v0, float v1, int q0, int q1, float w0,
+                                          float w1, uint32_t, uint32_t)
+    {
+        put<NT>(p0, v0);
+        put<NT>(p1, v1);
     }
 };
 
@@ -315,13 +334,22 @@ struct Codec<double, double, Q> {
     __device__ static inline double load(const double *p, int, double) { return *p; }
     __device__ static inline double load_nt(const double *p, int, double) { return __builtin_nontemporal_load(p); }
     __device__ static inline void store(double *p, double v, int, double) { *p = v; }
-    __device__ static inline void store_nt(double *p, double v, int, double) { __builtin_nontemporal_store(v, p); }
-    __device__ static inline void store_nt_sr(double *p, double v, int q, double w, uint32_t) { store_nt(p, v, q, w); }
-    __device__ static inline void store_nt_sr2(double *p0, double *p1, double v0, double v1, int q0, int q1, double w0,
-                                               double w1, uint32_t, uint32_t)
+    template <bool NT>
+    __device__ static inline void out(double *p, double v, int, double)
     {
-        store_nt(p0, v0, q0, w0);
-        store_nt(p1, v1, q1, w1);
+        put<NT>(p, v);
+    }
+    template <bool NT>
+    __device__ static inline void out_sr(double *p, double v, int q, double w, uint32_t)
+    {
+        put<NT>(p, v);
+    }
+    template <bool NT>
+    __device__ static inline void out_sr2(double *p0, double *p1, double v0, double v1, int q0, int q1, double w0,
+                                          double w1, uint32_t, uint32_t)
+    {
+        put<NT>(p0, v0);
+        put<NT>(p1, v1);
     }
 };
 
@@ -340,12 +368,14 @@ struct Codec<__half, float, Q> {
     {
         *p = __float2half_rn(dev_scaled<Q>(v, w, q));
     }
-    __device__ static inline void store_nt(__half *p, float v, int q, float w)
+    template <bool NT>
+    __device__ static inline void out(__half *p, float v, int q, float w)
     {
         __half h = __float2half_rn(dev_scaled<Q>(v, w, q));
-        __builtin_nontemporal_store(__half_as_ushort(h), (unsigned short *)p);
+        put<NT>((unsigned short *)p, __half_as_ushort(h));
     }
-    __device__ static inline void store_nt_sr(__half *p, float v, int q, float w, uint32_t r)
+    template <bool NT>
+    __device__ static inline void out_sr(__half *p, float v, int q, float w, uint32_t r)
     {
         typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
         h2_t h = {0, 0};
@@ -353,12 +383,13 @@ struct Codec<__half, float, Q> {
         const _Float16 e = h[0];
         unsigned short bits;
         __builtin_memcpy(&bits, &e, 2);
-        __builtin_nontemporal_store(bits, (unsigned short *)p);
+        put<NT>((unsigned short *)p, bits);
     }
     // two populations rounded into the two halves of one register (no register to clear
     // for the conversion's other half), stored from its low and high half
-    __device__ static inline void store_nt_sr2(__half *p0, __half *p1, float v0, float v1, int q0, int q1, float w0,
-                                               float w1, uint32_t r0, uint32_t r1)
+    template <bool NT>
+    __device__ static inline void out_sr2(__half *p0, __half *p1, float v0, float v1, int q0, int q1, float w0,
+                                          float w1, uint32_t r0, uint32_t r1)
     {
         typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
         // both halves are written below: start from the register of the random bits, which
@@ -370,8 +401,8 @@ struct Codec<__half, float, Q> {
         unsigned short b0, b1;
         __builtin_memcpy(&b0, &e0, 2);
         __builtin_memcpy(&b1, &e1, 2);
-        __builtin_nontemporal_store(b0, (unsigned short *)p0);
-        __builtin_nontemporal_store(b1, (unsigned short *)p1);
+        put<NT>((unsigned short *)p0, b0);
+        put<NT>((unsigned short *)p1, b1);
     }
 };
 
@@ -389,26 +420,29 @@ struct Codec<bf16_t, float, Q> {
     {
         p->bits = float_to_bf16(dev_scaled<Q>(v, w, q));
     }
-    __device__ static inline void store_nt(bf16_t *p, float v, int q, float w)
+    template <bool NT>
+    __device__ static inline void out(bf16_t *p, float v, int q, float w)
     {
-        __builtin_nontemporal_store(float_to_bf16(dev_scaled<Q>(v, w, q)), (unsigned short *)p);
+        put<NT>((unsigned short *)p, (unsigned short)float_to_bf16(dev_scaled<Q>(v, w, q)));
     }
-    __device__ static inline void store_nt_sr(bf16_t *p, float v, int q, float w, uint32_t r)
+    template <bool NT>
+    __device__ static inline void out_sr(bf16_t *p, float v, int q, float w, uint32_t r)
     {
         typedef short b2_t __attribute__((ext_vector_type(2)));
         b2_t h = {0, 0};
         h = __builtin_amdgcn_cvt_sr_bf16_f32(h, dev_scaled<Q>(v, w, q), r, false);
-        __builtin_nontemporal_store((unsigned short)h[0], (unsigned short *)p);
+        put<NT>((unsigned short *)p, (unsigned short)h[0]);
     }
-    __device__ static inline void store_nt_sr2(bf16_t *p0, bf16_t *p1, float v0, float v1, int q0, int q1, float w0,
-                                               float w1, uint32_t r0, uint32_t r1)
+    template <bool NT>
+    __device__ static inline void out_sr2(bf16_t *p0, bf16_t *p1, float v0, float v1, int q0, int q1, float w0,
+                                          float w1, uint32_t r0, uint32_t r1)
     {
         typedef short b2_t __attribute__((ext_vector_type(2)));
         b2_t h = __builtin_bit_cast(b2_t, r0);  // both halves are written below (as for FP16)
         h = __builtin_amdgcn_cvt_sr_bf16_f32(h, dev_scaled<Q>(v0, w0, q0), r0, false);
         h = __builtin_amdgcn_cvt_sr_bf16_f32(h, dev_scaled<Q>(v1, w1, q1), r1, true);
-        __builtin_nontemporal_store((unsigned short)h[0], (unsigned short *)p0);
-        __builtin_nontemporal_store((unsigned short)h[1], (unsigned short *)p1);
+        put<NT>((unsigned short *)p0, (unsigned short)h[0]);
+        put<NT>((unsigned short *)p1, (unsigned short)h[1]);
     }
 };
 
