@@ -97,11 +97,13 @@ __attribute__((amdgpu_waves_per_eu(Q == 27 ? kBatch27MinWaves<Real> : kBatch19Mi
 #define CELL_ALIGNED (PASS == 1)
 #define CELL_KEEP false
 #define CELL_COLL COLL
+#define CELL_EARLY false
             if constexpr (Q == 27) {
 #include "d3q27_cell.inc"
             } else {
 #include "d3q19_cell.inc"
             }
+#undef CELL_EARLY
 #undef CELL_COLL
 #undef CELL_KEEP
 #undef CELL_ALIGNED

@@ -425,6 +425,53 @@ __device__ inline Real wale_tau(const StepArgs<Real, Q> &a, long ic, int i, int 
     return wale_from_grad<Real>(dudx, dudy, dudz, dvdx, dvdy, dvdz, dwdx, dwdy, dwdz);
 }
 
+// What a cell needs beside its populations, loaded before anything is known of it (the latency
+// form of the step, PASS 4 of step19_kernel): its face velocity and, for WALE, the velocities of
+// its six neighbours, the cell itself in place of one outside the lattice.
+template <typename Real, bool WALE>
+struct EarlyLoads {
+    Real u0, v0, w0;
+    Real m[3][3], p[3][3];  // [component][axis]: the neighbour below and above
+};
+template <typename Real, bool WALE, int Q>
+__device__ __forceinline__ void early_loads(EarlyLoads<Real, WALE> &e, const StepArgs<Real, Q> &a, uint32_t ic, int i, int j,
+                                           int k)
+{
+    e.u0 = a.u0[ic];
+    e.v0 = a.v0[ic];
+    e.w0 = a.w0[ic];
+    if constexpr (WALE) {
+        const uint32_t sy = (uint32_t)a.nx, sz = sy * (uint32_t)a.ny;
+        const Real *const P[3] = {a.u_o, a.v_o, a.w_o};
+        const uint32_t up[3] = {i == a.nx - 1 ? ic : ic + 1u, j == a.ny - 1 ? ic : ic + sy, k == a.nz - 1 ? ic : ic + sz};
+        const uint32_t dn[3] = {i == 0 ? ic : ic - 1u, j == 0 ? ic : ic - sy, k == 0 ? ic : ic - sz};
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                e.p[c][x] = P[c][up[x]];
+                e.m[c][x] = P[c][dn[x]];
+            }
+    }
+}
+
+// wale_tau from the loaded neighbours: grad_comp's differences
+template <typename Real, int Q>
+__device__ __forceinline__ Real wale_tau_early(const StepArgs<Real, Q> &a, const EarlyLoads<Real, true> &e, int i, int j, int k,
+                                              Real u, Real v, Real w)
+{
+    auto diff = [](Real p, Real m, Real self, int pos, int n) {
+        return pos == 0 ? p - self : (pos == n - 1 ? self - m : Real(0.5) * (p - m));
+    };
+    auto diffz = [&](Real p, Real m, Real self) {
+        return a.nz == 1 ? Real(0) : (k == 0 ? p - p : (k == a.nz - 1 ? self - m : Real(0.5) * (p - m)));
+    };
+    return wale_from_grad<Real>(
+        diff(e.p[0][0], e.m[0][0], u, i, a.nx), diff(e.p[0][1], e.m[0][1], u, j, a.ny), diffz(e.p[0][2], e.m[0][2], u),
+        diff(e.p[1][0], e.m[1][0], v, i, a.nx), diff(e.p[1][1], e.m[1][1], v, j, a.ny), diffz(e.p[1][2], e.m[1][2], v),
+        diff(e.p[2][0], e.m[2][0], w, i, a.nx), diff(e.p[2][1], e.m[2][1], w, j, a.ny), diffz(e.p[2][2], e.m[2][2], w));
+}
+
 // reciprocal: one v_rcp_f32 in FP32 (<= 1 ulp), an exact quotient in FP64
 __device__ inline float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline double rcp(double x) { return 1.0 / x; }
@@ -701,9 +748,10 @@ __device__ __forceinline__ void outlet19(Real *ft, const S *fs, uint32_t fstride
 // on no other face) whose directions were pulled from the interior offsets already; only
 // the directions that cross its face (c_x = +1 at i = 0, c_x = -1 at i = nx - 1) are
 // streamed again.  The face conditions follow in either case.
-template <typename S, typename Real>
+// early: the face velocity, where it has been loaded already (else null).
+template <typename S, typename Real, typename E>
 __device__ __forceinline__ void face_cell(const Step19Args<Real> &a, Real *ft, uint32_t fl, long ic, int i, int j, int k,
-                                       Real omega, bool xonly)
+                                       Real omega, bool xonly, const E *early)
 {
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const S *fs = (const S *)a.fsrc;
@@ -758,7 +806,8 @@ __device__ __forceinline__ void face_cell(const Step19Args<Real> &a, Real *ft, u
 
     // fixedVelocityBC, kernel.cl:1397-1512
     if (corner == 0 && (b1 == BC_FIXEDVELOCITY || b2 == BC_FIXEDVELOCITY || b3 == BC_FIXEDVELOCITY)) {
-        const Real u0 = a.u0[ic], v0 = a.v0[ic], w0 = a.w0[ic];
+        const Real u0 = early ? early->u0 : a.u0[ic], v0 = early ? early->v0 : a.v0[ic],
+                   w0 = early ? early->w0 : a.w0[ic];
         if (b1 == BC_FIXEDVELOCITY && (i == 0 || i == nx - 1)) {
             const bool lo = (i == 0);
             Real rhow = zouhe_sum(ft, 0, lo) / (lo ? Real(1) - u0 : Real(1) + u0);
@@ -939,17 +988,45 @@ __device__ inline uint32_t face_blocks(const A &a)
     return merged_face_blocks(a.nface, blockDim.x);
 }
 
+// PASS 4 is the form for lattices whose waves are all resident at once and which wait for memory
+// one trip after another (kLatencyCells): it reads its arguments' cache lines together, then the
+// flags, the face velocity and WALE's neighbours beside the wave's class, where the others load
+// each when the one before has said that it is needed.  32^3 cavity 10.0 -> 8.3 us per step in
+// FP32, 11.2 -> 9.3 FP64, 9.4 -> 7.8 FP16 (a step that only streams, 2.7); of the 1.7 us, WALE's trip is 1.1.
+// Its registers (82 FP32, 146 FP64) cost occupancy, so that it ends where the waves no longer
+// fit: three waves per SIMD in FP32 (58^3 13.3 -> 11.5 us, but 64^3 13.1 -> 13.6), four with 16-bit
+// values (64^3 14.2 -> 12.4, 72^3 15.7 -> 19.1), one in FP64 (40^3 11.4 -> 9.8, the 192x24x24
+// box 11.5 -> 11.8).  D3Q27 gains a tenth in a cavity and loses a twentieth in a periodic box: it
+// has no such form.
+template <typename S>
+constexpr uint32_t kLatencyCells = 1024u * 64u * (sizeof(S) == 8 ? 1u : (sizeof(S) == 4 ? 3u : 4u));
+
 // Waves per SIMD the step kernel is held to: eight (64 VGPRs), which the compiler reaches
 // without spilling by interleaving each direction's pull address with its load; seven with
-// the interpolated bounce-back, whose groups of links spill at eight; FP64 as the compiler
-// chooses.
-template <typename S, typename Real, int SGS, bool IBB>
-constexpr int kStep19MinWaves = sizeof(Real) == 8 ? 1 : (IBB ? 7 : 8);
+// the interpolated bounce-back, whose groups of links spill at eight; FP64 and the latency form as
+// the compiler chooses.
+template <typename S, typename Real, int SGS, bool IBB, int PASS>
+constexpr int kStep19MinWaves = (sizeof(Real) == 8 || PASS == 4) ? 1 : (IBB ? 7 : 8);
+
+// reads one word of every 64 bytes of the launch arguments: the scalar loads that take them
+// where they are used then find them in the scalar cache, instead of missing it once per line
+// along the kernel (0.4 us of a small lattice's step)
+template <typename A>
+__device__ __forceinline__ void touch_args()
+{
+    typedef const __attribute__((address_space(4))) uint32_t const_u32;
+    const_u32 *p = (const_u32 *)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t x = 0;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(A) / 4; i += 16) x |= p[i];
+    asm volatile("" ::"s"(x));
+}
 
 template <typename S, typename Real, int SGS, bool IBB = false, int AA = 0, int PASS = 0>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStep19MinWaves<S, Real, SGS, IBB>, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStep19MinWaves<S, Real, SGS, IBB, PASS>, 8)))
 step19_kernel(const Step19Args<Real> a)
 {
+    if constexpr (PASS == 4) touch_args<Step19Args<Real>>();
     const uint32_t nfb = (PASS == 3) ? face_blocks(a) : 0u;
     const bool face_wg = (PASS == 2) || (PASS == 3 && blockIdx.x < nfb);
     uint32_t icu;
@@ -973,7 +1050,9 @@ step19_kernel(const Step19Args<Real> a)
 #define CELL_PURE_OK (AA == 0 && !face_wg)
 #define CELL_ALIGNED (!face_wg && a.wave_runs)
 #define CELL_KEEP a.keep
+#define CELL_EARLY (PASS == 4)
 #include "d3q19_cell.inc"
+#undef CELL_EARLY
 #undef CELL_KEEP
 #undef CELL_ALIGNED
 #undef CELL_PURE_OK

@@ -57,6 +57,8 @@ void launch_step(const StepArgs<Real, Q> &a, unsigned grid, int block, hipStream
             hipLaunchKernelGGL((step19_kernel<S, Real, SGS, false, 0, 1>), dim3(grid), dim3(block), 0, st, a);
             if (fgrid)
                 hipLaunchKernelGGL((step19_kernel<S, Real, SGS, false, 0, 2>), dim3(fgrid), dim3(block), 0, st, a);
+        } else if (a.N <= kLatencyCells<S>) {
+            hipLaunchKernelGGL((step19_kernel<S, Real, SGS, false, 0, 4>), dim3(grid), dim3(block), 0, st, a);
         } else {
             hipLaunchKernelGGL((step19_kernel<S, Real, SGS, false, 0, 0>), dim3(grid), dim3(block), 0, st, a);
         }
