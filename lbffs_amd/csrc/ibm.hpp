@@ -82,12 +82,26 @@ __device__ inline uint32_t lanes_below(uint64_t mask)
 }
 
 // k_Gwall (K19:3648-3716) and k_Gibm (K19:3718-3779) with a summing spread; cells touched this
-// step are listed once.  What bounds it is latency (a few hundred waves in all): the 24
-// velocities, then the 24 adds and 8 stamps go out together (a corner outside the lattice reads
-// corner 0, weightless), and a wave takes its list slots with one add to the counter.  One
-// corner at a time, with a returning atomic and an add to the counter each, in two kernels,
-// 6400 markers took 30 us per step, now 19 (what is left is the atomics themselves).
+// step are listed once.  What bounds it is latency and the adds to memory: markers lie closer
+// than a cell, so that 64 of them in a row share their 512 corners several times over.  Where the box
+// of a wave's corners has no more cells than that (markers listed along a surface), the wave sums
+// them by cell in LDS and every cell touched takes one stamp and three adds to memory; otherwise
+// each corner goes there itself.  The 24 velocities of a marker are
+// loaded together (a corner outside the lattice reads corner 0, weightless), and a wave takes its
+// list slots with one add to the counter.  One corner at a time,
+// with a returning atomic and an add to the counter each, in two kernels, 6400 markers of a ring
+// took 30 us per step; with their adds batched 19, with the box 8 (192x96x64 FP32 step with markers
+// 63.0 -> 52.4 us).  Markers in no order (6400 over 96x64x64: 50 us either way) keep the direct adds.
 constexpr int kIbmBlock = 64;
+constexpr int kIbmBox = 8 * kIbmBlock;  // cells of the largest box summed in LDS
+// least value over the wave's lanes (a full wave)
+__device__ inline int wave_min(int v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d));
+    return v;
+}
+
 template <typename Real>
 __global__ void __launch_bounds__(kIbmBlock)
     ibm_spread_move_kernel(int n, Real *xyz, int nx, int ny, int nz, const Real *u, const Real *v, const Real *w,
@@ -96,15 +110,16 @@ __global__ void __launch_bounds__(kIbmBlock)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = p < n;
-    Real x = 0, y = 0, z = 0;
-    uint32_t ib[8], fresh = 0;  // the corners this marker is the first to touch in this step
+    __shared__ Real G[3][kIbmBox];
+    __shared__ uint32_t touched[kIbmBox];
+    Real x = 0, y = 0, z = 0, gx = 0, gy = 0, gz = 0, d[8];
+    uint32_t ib[8], in = 0;  // corners; those inside the lattice
+    int i = 0, j = 0, k = 0;
     if (active) {
         x = xyz[3 * p];
         y = xyz[3 * p + 1];
         z = xyz[3 * p + 2];
-        const int i = (int)x, j = (int)y, k = (int)z;  // truncation (K19:3671-3673)
-        Real d[8];
-        uint32_t in = 0;
+        i = (int)x, j = (int)y, k = (int)z;  // truncation (K19:3671-3673)
         if (i >= 0 && i < nx && j >= 0 && j < ny && k >= 0 && k < nz) {
 #pragma unroll
             for (int b = 0; b < 8; b++) in |= box_corner(b, i, j, k, nx, ny, nz, x, y, z, ib[b], d[b]) ? 1u << b : 0u;
@@ -131,14 +146,55 @@ __global__ void __launch_bounds__(kIbmBlock)
         Real U[3];
 #pragma unroll
         for (int a = 0; a < 3; a++) U[a] = m.trans[a] + F.r * m.omega * F.e2[a];
-        const Real gx = U[0] - ui, gy = U[1] - vi, gz = U[2] - wi;
+        gx = U[0] - ui, gy = U[1] - vi, gz = U[2] - wi;
         Gm[p] = gx;
         Gm[n + p] = gy;
         Gm[2 * n + p] = gz;
-        uint32_t old[8];
+    }
+    // the box of the wave's corners (a marker outside the lattice takes no part)
+    const int lox = wave_min(in ? i : nx), loy = wave_min(in ? j : ny), loz = wave_min(in ? k : nz);
+    const int bx = 2 - lox - wave_min(in ? -i : 0), by = 2 - loy - wave_min(in ? -j : 0), bz = 2 - loz - wave_min(in ? -k : 0);
+    const bool any = __ballot(in != 0) != 0;
+    uint32_t ic[8], old[8];
 #pragma unroll
-        for (int b = 0; b < 8; b++)
+    for (int b = 0; b < 8; b++) old[b] = stamp;
+    if (any && (long)bx * by * bz <= kIbmBox) {
+        const uint32_t cells = (uint32_t)(bx * by * bz);
+        for (uint32_t e = threadIdx.x; e < cells; e += kIbmBlock) {
+            touched[e] = 0;
+            G[0][e] = G[1][e] = G[2][e] = Real(0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            if (!((in >> b) & 1u)) continue;
+            const int di = (b == 1 || b == 4 || b == 5 || b == 7) ? 1 : 0;
+            const int dj = (b == 2 || b == 4 || b == 6 || b == 7) ? 1 : 0;
+            const int dk = (b == 3 || b == 5 || b == 6 || b == 7) ? 1 : 0;
+            const int e = (i + di - lox) + bx * ((j + dj - loy) + by * (k + dk - loz));
+            touched[e] = 1;
+            atomicAdd(&G[0][e], gx * d[b]);
+            atomicAdd(&G[1][e], gy * d[b]);
+            atomicAdd(&G[2][e], gz * d[b]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const uint32_t e = (uint32_t)b * kIbmBlock + threadIdx.x;
+            if (e >= cells || !touched[e]) continue;
+            const uint32_t t = e / (uint32_t)bx, di = e - t * (uint32_t)bx, dk = t / (uint32_t)by, dj = t - dk * (uint32_t)by;
+            ic[b] = (lox + di) + (uint32_t)nx * ((loy + dj) + (uint32_t)ny * (loz + dk));
+            old[b] = atomicExch(&mark[ic[b]], stamp);
+            atomicAdd(&Gx[ic[b]], G[0][e]);
+            atomicAdd(&Gy[ic[b]], G[1][e]);
+            atomicAdd(&Gz[ic[b]], G[2][e]);
+        }
+    } else {
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            ic[b] = ib[b];
             if ((in >> b) & 1u) old[b] = atomicExch(&mark[ib[b]], stamp);
+        }
 #pragma unroll
         for (int b = 0; b < 8; b++)
             if ((in >> b) & 1u) {
@@ -146,23 +202,20 @@ __global__ void __launch_bounds__(kIbmBlock)
                 atomicAdd(&Gy[ib[b]], gy * d[b]);
                 atomicAdd(&Gz[ib[b]], gz * d[b]);
             }
-#pragma unroll
-        for (int b = 0; b < 8; b++)
-            if ((in >> b) & 1u) fresh |= old[b] != stamp ? 1u << b : 0u;
     }
-    // list slots: one add to the counter per wave, corner by corner in lane order after it
+    // list slots: one add to the counter per wave, group by group in lane order after it
     uint32_t total = 0;
 #pragma unroll
-    for (int b = 0; b < 8; b++) total += (uint32_t)__popcll(__ballot((fresh >> b) & 1u));
+    for (int b = 0; b < 8; b++) total += (uint32_t)__popcll(__ballot(old[b] != stamp));
     int base = 0;
-    if (total && (threadIdx.x & 63) == 0) base = atomicAdd(count, (int)total);
+    if (total && threadIdx.x == 0) base = atomicAdd(count, (int)total);
     base = __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
     for (int b = 0; b < 8; b++) {
-        const uint64_t mask = __ballot((fresh >> b) & 1u);
-        if ((fresh >> b) & 1u) {
+        const uint64_t mask = __ballot(old[b] != stamp);
+        if (old[b] != stamp) {
             const int slot = base + (int)lanes_below(mask);
-            if (slot < cap) list[slot] = (int)ib[b];
+            if (slot < cap) list[slot] = (int)ic[b];
         }
         base += __popcll(mask);
     }
