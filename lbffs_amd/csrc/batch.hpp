@@ -62,9 +62,11 @@ __host__ inline unsigned batch_grid(unsigned grid, uint32_t n)
     return g >= n ? n : g;
 }
 
-// Waves per SIMD the D3Q19 block-table pass is held to: eight with WALE (64 VGPRs, no spill;
+// Waves per SIMD the D3Q19 block-table pass is held to: eight with WALE (64 VGPRs;
 // the ensemble's step 6.63 -> 6.22 ms), seven without a sub-grid model, where eight loads
-// fewer populations in flight and ran slower (5.30 -> 5.92 ms).
+// fewer populations in flight and ran slower (5.30 -> 5.92 ms).  The face
+// pass and the interpolated bounce-back run at five, which hold their loads in flight without
+// spilling (93-96 VGPRs); FP64 as the compiler chooses.
 template <int SGS, bool IBB, int PASS, typename Real>
 constexpr int kBatch19MinWaves = sizeof(Real) == 8 ? 1 : ((IBB || PASS != 1) ? 5 : (SGS == 0 ? 8 : 7));
 

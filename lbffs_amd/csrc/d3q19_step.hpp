@@ -982,6 +982,7 @@ __device__ __forceinline__ bool x_face19(const Step19Args<Real> &a, Real *ft, ui
 // first and run beside the interior ones).
 // (rounded up to a multiple of 8, so that the blocks after them keep their hardware XCD
 // order; the work-groups past the list end at once)
+// PASS 4 runs every cell as 0 does, in the form for small lattices (kLatencyCells).
 template <typename A>
 __device__ inline uint32_t face_blocks(const A &a)
 {
