@@ -97,7 +97,7 @@ __attribute__((amdgpu_waves_per_eu(Q == 27 ? kBatch27MinWaves<Real> : kBatch19Mi
 #define CELL_SKIP_FACE (PASS == 1)
 #define CELL_PURE_OK (PASS == 1)
 #define CELL_ALIGNED (PASS == 1)
-#define CELL_KEEP false
+#define CELL_KEEP a.keep
 #define CELL_COLL COLL
 #define CELL_EARLY false
             if constexpr (Q == 27) {

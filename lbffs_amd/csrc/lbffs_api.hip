@@ -584,11 +584,12 @@ uint32_t ytile_rows(const lbffs_ctx *c)
 // (144x150x73 FP32 55.4 against 56.2, 160x191x86 FP16 66.4 against 70.4).  Below 80 MB the write-back
 // of the L2s at the end of every launch takes back what the hits give (64x72x34 FP32 11.0
 // streamed, 11.6 kept; D3Q27 80x84x41 FP32 17.6 and 18.4).
-bool fits_cache(const lbffs_ctx *c)
+double step_bytes(const lbffs_ctx *c)
 {
-    const double bytes = (double)c->N * (2.0 * c->d.q * c->store_size + 8.0 * c->real_size + 2.0);
-    return c->d.streaming != LBFFS_STREAM_AA && bytes >= 80e6 && bytes <= 256.0 * (1 << 20);
+    return (double)c->N * (2.0 * c->d.q * c->store_size + 8.0 * c->real_size + 2.0);
 }
+bool cache_holds(double bytes) { return bytes >= 80e6 && bytes <= 256.0 * (1 << 20); }
+bool fits_cache(const lbffs_ctx *c) { return c->d.streaming != LBFFS_STREAM_AA && cache_holds(step_bytes(c)); }
 
 // whether the step kernels of this lattice read its per-wave flag summary: the summary
 // names aligned runs of 64 cells, which a wave covers when its cells are consecutive (the
@@ -1111,6 +1112,12 @@ template <typename S, typename Real, int Q>
 int batch_steps_q(lbffs_batch *b, int nsteps, const lbffs_step_params *params)
 {
     const int cur0 = b->ctx[0]->cur;
+    // The lattices of a batch share the cache (fits_cache).  10 lattices of edge 24-64, 124 MB FP16:
+    // 48.5 -> 45.2 us per step, 210 MB FP32 57.5 -> 50.5, 244 MB FP64 66.0 -> 61.4, D3Q27 187 MB BF16
+    // 91.7 -> 74.5; 16-bit batches end earlier (240 MB FP16 76.1 -> 78.9).
+    double bytes = 0;
+    for (const lbffs_ctx *c : b->ctx) bytes += step_bytes(c);
+    const bool keep = cache_holds(bytes) && (sizeof(S) != 2 || bytes <= 224e6);
     for (int v = 0; v < 4; v++) {
         const int p = v & 1, last = v >> 1;
         b->args_host[v].assign(b->ctx.size() * sizeof(StepArgs<Real, Q>), 0);
@@ -1134,6 +1141,7 @@ int batch_steps_q(lbffs_batch *b, int nsteps, const lbffs_step_params *params)
             a.rho_all = a.aux_all;
             a.step = c->nstep;  // + the device counter of steps within this call
             a.step_ctr = b->ctr;
+            a.keep = (keep && !(c->tune & TUNE_NT_STORE)) ? 1 : 0;
         }
         HIP_TRY(hipMemcpy(b->args_dev[v], b->args_host[v].data(), b->args_host[v].size(), hipMemcpyHostToDevice));
     }
