@@ -14,6 +14,18 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs through the HIP library)")
 
 
+def pytest_collection_modifyitems(items):
+    """The GPU tests that run the reference's own kernels need their builds, which the oracle's
+    makefile makes where the reference's sources are present."""
+    ref = os.path.join(ROOT, "oracle", "_ref")
+    if all(os.path.exists(os.path.join(ref, f)) for f in ("kernel19.co", "kernel27.co")):
+        return
+    skip = pytest.mark.skip(reason="the reference's kernels are not built (its sources are absent)")
+    for item in items:
+        if item.get_closest_marker("gpu") and "_reference_" in item.name:
+            item.add_marker(skip)
+
+
 def rel_l2(a, b):
     a = np.asarray(a, np.float64)
     b = np.asarray(b, np.float64)
